@@ -44,15 +44,19 @@ int vllm_mi355x_abi_version(void);
 /* ---- EXL3 ---------------------------------------------------------------- */
 
 /*
- * FP32 workspace elements exl3_linear_out needs for calls of up to max_rows
- * rows of a padded_in x padded_out matrix: the larger of the small-M path's
- * K-split partial sums, min(max_rows, 8) * splits * padded_out (splits =
- * padded_in / 128 / blocks, with the automatic blocks per workgroup, at most
- * 32 where the shape allows), and, above exl3_linear_prefill_rows() rows,
- * the large-M path's max_rows * (padded_in + 1) (FP16 high/low activations,
- * one row exponent per row).  The two paths never run in one call.  Returns
- * -1 (with an error message) for a negative row count or padded sizes that
- * are not positive multiples of 128.
+ * FP32 workspace elements exl3_linear_out uses for calls of up to max_rows
+ * rows of a padded_in x padded_out matrix: the largest, over those row
+ * counts, of the small-M path's K-split partial sums, min(rows, 8) * splits *
+ * padded_out (splits = padded_in / 128 / blocks, with the automatic blocks
+ * per workgroup, at most 32 where the shape allows), and the tile GEMM's
+ * rows * (padded_in + 1) (FP16 high/low activations, one row exponent per
+ * row) and partial sums (its K splits * rows * padded_out, counted up to 8M
+ * floats in all).  The two paths never run in one call.  exl3_linear_out
+ * accepts less, down to the small-M partial sums and, above
+ * exl3_linear_prefill_rows() rows, rows * (padded_in + 1): the tile GEMM then
+ * splits K less, and calls of up to 32 rows run in chunks of 8.  Returns -1
+ * (with an error message) for a negative row count or padded sizes that are
+ * not positive multiples of 128.
  * Replaces _exl3_C::linear_workspace_size (csrc/exl3/dense.cu:72-78).
  */
 int64_t exl3_linear_workspace_size(int64_t max_rows, int64_t padded_in, int64_t padded_out);
@@ -85,8 +89,10 @@ int exl3_linear_out_scratch(const void* x, int x_dtype, int64_t rows, int64_t x_
 int64_t exl3_linear_scratch_rows(int64_t padded_in, int64_t padded_out);
 
 /*
- * The row count above which exl3_linear_out runs the large-M (prefill) GEMM;
- * up to it, the small-M kernel in chunks of 8 rows.  The reference's routing
+ * The row count above which exl3_linear_out always runs a many-row GEMM.  Up
+ * to it: the small-M kernel for 8 rows; above 8, the tile GEMM where it
+ * applies (at least 1024 inputs, a 16-byte aligned trellis, a workspace with
+ * room), else the small-M kernel in chunks of 8 rows.  The reference's routing
  * question _exl3_C::linear_prefill_applies (vllm_sm80/kernels/exl3/
  * dense_prefill_tc.py:57-80) answers from it.
  */
@@ -104,8 +110,8 @@ int exl3_linear_prefill_rows(void);
  *   suh      fp16 [suh_numel == padded_in], svh fp16 [svh_numel == padded_out]
  *   bits_x2  2..16 with codebook 1 (mcg, even rates) or 2 (mul1, also 3/5/7)
  *   out      [rows][logical_out] of out_dtype (VQ_BF16, VQ_FP16 or VQ_FP32)
- *   workspace FP32, >= exl3_linear_workspace_size(rows, ...) elements,
- *            16-byte aligned, overlapping no other argument.
+ *   workspace FP32, exl3_linear_workspace_size(rows, ...) elements (or
+ *            fewer, see there), 16-byte aligned, overlapping no other argument.
  * The weights are decoded bit-exactly; the products are summed in FP32 on
  * the matrix cores, with the activations split into FP16 high and low
  * parts (about 22 significant bits, the activation precision of the

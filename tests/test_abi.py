@@ -181,3 +181,22 @@ def test_moe_launch_rows_keeps_offsets_in_32_bits():
     assert rows == (2 ** 31 - 1) // (4 * 7168 * 9)
     assert rows * 9 * 7168 * 4 <= 2 ** 31 - 1 < (rows + 1) * 9 * 7168 * 4
     assert ops.moe_launch_rows(100, 300, 8) == (2 ** 31 - 1) // (4 * 384 * 8)
+
+
+@pytest.mark.parametrize("k,n", [(1024, 128), (4096, 4096), (4096, 14336), (14336, 512), (128, 256)])
+def test_linear_workspace_size_grows_with_rows_and_keeps_the_row_chunks(k, n):
+    """The size with room for the K splits never shrinks as rows grow, is at
+    least the unsplit path's need, and passes the fixed 8M-float scratch
+    only where that need does: callers that cut their rows to the scratch cut
+    them as before."""
+    from vllm_mi355x import _native
+    lib = _native.load()
+    scratch = 8 << 20
+    limit = scratch // (k + 1)
+    rows = sorted({1, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 300, 1024, limit, limit + 1, 2 * limit})
+    sizes = [lib.exl3_linear_workspace_size(r, k, n) for r in rows]
+    assert sizes == sorted(sizes)
+    for r, size in zip(rows, sizes):
+        if r > 32:
+            assert size >= r * (k + 1)
+            assert (size <= scratch) == (r * (k + 1) <= scratch)

@@ -569,3 +569,40 @@ def test_many_captures_keep_the_fused_finish(ops, device):
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
     del graphs
+
+
+# (k, n, rows): heights around every tile's (32, 64 and 128 rows and whole
+# 16-row blocks of them), K ranges that split unevenly (9 and 17 blocks), a
+# last column tile of 128 columns, a matrix below the 9-row minimum width
+SPLIT_SHAPES = [(1152, 384, 9), (1152, 384, 16), (2176, 256, 17), (1152, 384, 32), (1152, 384, 33),
+                (2176, 128, 64), (1152, 384, 65), (1152, 640, 97), (2176, 384, 128), (1152, 384, 129),
+                (1152, 256, 273), (896, 384, 20)]
+
+
+@pytest.mark.parametrize("shape", SPLIT_SHAPES)
+@pytest.mark.parametrize("bits_x2,codebook", [(8, 2), (3, 2), (12, 1)])
+def test_tile_splits_match_oracle(ops, device, shape, bits_x2, codebook):
+    """The K-split tile GEMM against the oracle at the FP32 bar (the same
+    activations and products, FP32 sums in another order), with the
+    workspace the size function gives, and with the smallest one accepted
+    (fewer splits or none), which must agree within two such bars."""
+    k, n, rows = shape
+    print(f"tile splits {shape} bits_x2={bits_x2} codebook={codebook}", flush=True)
+    rng = np.random.default_rng(k + n + rows + bits_x2)
+    trellis, suh, svh = random_matrix(rng, k, n, bits_x2)
+    x, code = random_acts(rng, rows, k - 5, "fp16")
+    t, u, v, xt = _dev(trellis, device), _dev(suh, device), _dev(svh, device), _dev(x, device)
+    full = ops.linear_workspace_size(rows, k, n)
+    least = rows * (k + 1) if rows > 32 else ops.linear_workspace_size(8, k, n)
+    got = []
+    for size in (full, least):
+        # (the guard past the workspace's end must stay untouched)
+        ws = torch.full((size + 64,), float("nan"), dtype=torch.float32, device=device)
+        out = torch.empty(rows, n - 3, dtype=torch.float32, device=device)
+        ops.linear_out(xt, t, u, v, bits_x2, codebook, k - 5, n - 3, out, ws[:size])
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(ws[size:]).all())
+        got.append(_out_np(out))
+    want = O.linear_out(x, code, trellis, suh, svh, bits_x2, codebook, n - 3, O.FP32)
+    for g in got:
+        _assert_fp32_close(g, want, f"{shape}")

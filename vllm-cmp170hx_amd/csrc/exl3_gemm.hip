@@ -1,8 +1,10 @@
-// EXL3 dense linear for many rows (prefill), gfx950.
+// EXL3 dense linear for many rows (more than 8 on the tile GEMM), gfx950.
 //
 // Two launches on the caller's stream, where the reference's operator has
 // three (csrc/exl3/dense.cu:115-148: linear_input, GEMM, linear_output); the
-// GEMM runs on the matrix cores and applies the output transform itself:
+// GEMM runs on the matrix cores and applies the output transform itself, or,
+// where its K range is split over workgroups, a third launch (tile_output)
+// adds the splits and applies it:
 //  1. prefill_input: one workgroup per row forms t = H128(x * suh) over the
 //     whole row, picks a per-row power-of-two scale from the row maximum, and
 //     writes t as FP16 high and low parts (t * 2^e = hi + lo, ~22 bits), in
@@ -31,9 +33,11 @@
 //     H128 over each 128-column block, times svh, rounded to the output dtype.
 //
 // Workspace (FP32 elements): rows x padded_in floats holding the FP16 rows
-// above, and one int row exponent per row after them.
+// above, one int row exponent per row after them, then (from the next 16
+// bytes on) the partial sums of the K splits, rows x padded_out floats each.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <climits>
 #include <type_traits>
@@ -60,10 +64,13 @@ constexpr int kLdsK = kBK + 8;      // LDS row stride in halves (80 bytes)
 
 // ---- 1. activations ----------------------------------------------------------
 
-// One workgroup (256 threads) per row.  A wavefront forms four 128-input
-// blocks at a time (group G: blocks 4 G .. 4 G + 3, one per 16-lane row,
-// eight consecutive inputs a lane, H128 in registers and DPP); wavefront w
-// takes groups w, w + 4, ..., the first kCache of them kept in registers.
+// One workgroup of kWavesRow wavefronts per row.  A wavefront forms four
+// 128-input blocks at a time (group G: blocks 4 G .. 4 G + 3, one per 16-lane
+// row, eight consecutive inputs a lane, H128 in registers and DPP); wavefront w
+// takes groups w, w + kWavesRow, ..., the first kCache of them kept in
+// registers.  A row's chain of loads, transform and maximum sets the time
+// of a call of few rows: 20 rows of 14336 inputs take 15.4 us with four
+// wavefronts a row (seven groups each) and under 6 with sixteen.
 // Pass 1 finds the row maximum of |t|, pass 2 writes the scaled high parts
 // (and the low parts when `lo`: the GEMM reads them) as dword pairs; groups past the register cache are formed again
 // (the same operations, so the same values).  Inputs past logical_in form
@@ -76,8 +83,8 @@ __device__ __forceinline__ int64_t operand_order(int64_t k) {
   return (k & ~int64_t(31)) + g * 8 + slot;
 }
 
-template <int kCache>
-__global__ __launch_bounds__(256) void prefill_input(const void* __restrict__ x, int x_dtype,
+template <int kCache, int kWavesRow>
+__global__ __launch_bounds__(64 * kWavesRow) void prefill_input(const void* __restrict__ x, int x_dtype,
                                                      int64_t logical_in, int64_t padded_in,
                                                      const uint16_t* __restrict__ suh,
                                                      _Float16* __restrict__ act,
@@ -125,15 +132,15 @@ __global__ __launch_bounds__(256) void prefill_input(const void* __restrict__ x,
   float mx = 0.0f;
   float c[kCache][8];
 #pragma unroll
-  for (int i = 0; i < kCache; ++i) form(min(int64_t(wave + 4 * i), groups - 1), c[i]);
+  for (int i = 0; i < kCache; ++i) form(min(int64_t(wave + kWavesRow * i), groups - 1), c[i]);
 #pragma unroll
   for (int i = 0; i < kCache; ++i) {
-    if (wave + 4 * i < groups && live(wave + 4 * i)) {
+    if (wave + kWavesRow * i < groups && live(wave + kWavesRow * i)) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(c[i][j]));
     }
   }
-  for (int64_t G = wave + 4 * kCache; G < groups; G += 4) {
+  for (int64_t G = wave + kWavesRow * kCache; G < groups; G += kWavesRow) {
     float v[8];
     form(G, v);
     if (live(G)) {
@@ -167,9 +174,9 @@ __global__ __launch_bounds__(256) void prefill_input(const void* __restrict__ x,
   };
 #pragma unroll
   for (int i = 0; i < kCache; ++i) {
-    if (wave + 4 * i < groups && live(wave + 4 * i)) store8(first_k(wave + 4 * i), c[i]);
+    if (wave + kWavesRow * i < groups && live(wave + kWavesRow * i)) store8(first_k(wave + kWavesRow * i), c[i]);
   }
-  for (int64_t G = wave + 4 * kCache; G < groups; G += 4) {
+  for (int64_t G = wave + kWavesRow * kCache; G < groups; G += kWavesRow) {
     float v[8];
     form(G, v);
     if (live(G)) store8(first_k(G), v);
@@ -421,15 +428,15 @@ int launch_gemm(bool aligned, const PrefillArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-int launch_tile_gemm(int64_t bits_x2, int64_t codebook, bool moe, bool lo, const TileArgs& a, dim3 grid,
-                     hipStream_t stream) {
+int launch_tile_gemm(int64_t bits_x2, int64_t codebook, bool moe, bool lo, int blocks, const TileArgs& a,
+                     dim3 grid, hipStream_t stream) {
   const int index = format_index(int(bits_x2), int(codebook));
   if (index < 0 || !known_format(bits_x2, codebook) || !tile_rate(bits_x2)) {
     return vq::fail("Unsupported EXL3 rate/codebook combination");
   }
   switch (index % kTileParts) {
 #define VQ_PART(P) \
-  case P: return tile_launch_part<P>(bits_x2, codebook, moe, lo, a, grid, stream);
+  case P: return tile_launch_part<P>(bits_x2, codebook, moe, lo, blocks, a, grid, stream);
     VQ_PART(0) VQ_PART(1) VQ_PART(2) VQ_PART(3)
 #undef VQ_PART
   }
@@ -442,42 +449,147 @@ namespace {
 std::atomic<int> g_tile_fp16_only{0};
 std::atomic<int> g_prefill_kernel{0};
 
+// Workgroups a split grid is cut into at most, and the shortest K range of a
+// split in 128-input blocks.  A call whose tiles leave CUs idle splits K until
+// it has about one workgroup per CU, two for tiles of 32 rows (a short step
+// leaves latency for a second workgroup to fill); beyond that the partial sums
+// cost more than they win.  Measured (us per call, 4 bits, 1 / 4 / 8 / 16 / 32
+// splits): 14336 x 4096 at 77 rows (16 tiles) 293 / 84 / 56 / 43 / 54 before
+// the finish read its splits in parallel; 4096 x 4096 at 200 rows (32
+// tiles) 122 / 47 / 38 / 45 / 45; 4096 x 14336 at 20 rows (56 tiles) 76 / 30 /
+// 29 / 31 / 52; at 64 rows 88 / 38 / 38 / 38 / 38.
+constexpr int64_t kSplitGrid = 256;
+constexpr int64_t kSplitGridLow = 512;
+constexpr int64_t kSplitMinBlocks = 2;
+
+// The finish of a K-split tile GEMM: one workgroup sums four rows of one
+// 128-column block, wavefront w over the splits w, w + 4, ... (lane (q, l)
+// row q's columns 8 l .. 8 l + 7, eight splits' loads in flight), the four
+// sums added in wavefront order; then H128, times svh, rounded to the output
+// dtype.
+__global__ __launch_bounds__(256) void tile_output(const float* __restrict__ partial, int splits, int64_t rows,
+                                                   int64_t np, const uint16_t* __restrict__ svh,
+                                                   int64_t logical_out, void* out, int out_dtype) {
+  __shared__ f32x4_t sums[3][2][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int q = lane >> 4;
+  const int l = lane & 15;
+  const int64_t blocks = np / 128;
+  const int64_t row = int64_t(blockIdx.x) / blocks * 4 + q;
+  const int64_t c0 = int64_t(blockIdx.x) % blocks * 128 + 8 * l;
+  const float* p = partial + min(row, rows - 1) * np + c0;
+  const int64_t stride = rows * np;
+  uint16_t scales[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) scales[j] = svh[c0 + j];
+  f32x4_t v0 = {0.0f, 0.0f, 0.0f, 0.0f}, v1 = v0;
+  for (int s0 = wave; s0 < splits; s0 += 32) {
+    f32x4_t t0[8], t1[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float* src = p + min(s0 + 4 * u, splits - 1) * stride;
+      t0[u] = *reinterpret_cast<const f32x4_t*>(src);
+      t1[u] = *reinterpret_cast<const f32x4_t*>(src + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (s0 + 4 * u < splits) {
+        v0 += t0[u];
+        v1 += t1[u];
+      }
+    }
+  }
+  if (wave > 0) {
+    sums[wave - 1][0][lane] = v0;
+    sums[wave - 1][1][lane] = v1;
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 0; w < 3; ++w) {
+    v0 += sums[w][0][lane];
+    v1 += sums[w][1][lane];
+  }
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float a = v0[j], b = v1[j];
+    v[j] = a;
+    v[4 + j] = b;
+  }
+  vq::h128_rows(v, l);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] *= vq::f16_to_f32(scales[j]);
+  if (row < rows) vq::store8_act(out, out_dtype, row * logical_out + c0, v, logical_out - c0);
+}
+
 }  // namespace
 
 bool tile_fp16_only() { return g_tile_fp16_only.load() != 0; }
 
+bool tile_applies(const void* trellis, int64_t tiles_k, int64_t tiles_n, int64_t bits_x2, int64_t rows) {
+  return g_prefill_kernel.load() != 1 && tile_rate(bits_x2) && (reinterpret_cast<uintptr_t>(trellis) & 15) == 0 &&
+         tiles_k * tiles_n * 16 * bits_x2 <= INT_MAX && rows * 64 * tiles_k <= INT_MAX;
+}
+
+TilePlan plan_tile(int64_t rows, int64_t kp, int64_t np) {
+  TilePlan p{};
+  p.blocks = rows <= 32 ? 2 : (rows <= 64 ? 4 : kTileBlocks);
+  // rows spread evenly over the row tiles, in whole 16-row blocks
+  p.row_tiles = (rows + 16 * p.blocks - 1) / (16 * p.blocks);
+  p.tile_rows = int(((rows + p.row_tiles - 1) / p.row_tiles + 15) / 16 * 16);
+  p.row_tiles = (rows + p.tile_rows - 1) / p.tile_rows;
+  const int64_t tiles = p.row_tiles * ((np + kTileCols - 1) / kTileCols);
+  const int64_t wanted = p.blocks == 2 ? kSplitGridLow : kSplitGrid;
+  const int64_t k_blocks = kp / 128;
+  const int64_t splits = std::max<int64_t>(1, std::min(wanted / tiles, k_blocks / kSplitMinBlocks));
+  // whole 128-input blocks a split: no more splits than the longest needs
+  const int64_t per_split = (k_blocks + splits - 1) / splits;
+  p.splits = int((k_blocks + per_split - 1) / per_split);
+  return p;
+}
+
 int prefill_linear(const void* x, int x_dtype, int64_t rows, const uint8_t* trellis,
                    int64_t tiles_k, int64_t tiles_n, const uint16_t* suh, const uint16_t* svh,
                    int bits_x2, int codebook, int64_t logical_in, int64_t logical_out, void* out,
-                   int out_dtype, float* workspace, hipStream_t stream) {
+                   int out_dtype, float* workspace, int64_t workspace_numel, hipStream_t stream) {
   const int64_t kp = tiles_k * 16;
   const int64_t np = tiles_n * 16;
   if (rows > 65535 * int64_t(kTileRows)) return vq::fail("EXL3 linear has too many rows");
   _Float16* act = reinterpret_cast<_Float16*>(workspace);
   int* row_exp = reinterpret_cast<int*>(workspace + rows * kp);
-  // the tile GEMM: a 16-byte aligned trellis (LDS-DMA), 32-bit buffer
-  // offsets over the matrix and the activations; under
-  // exl3_set_tile_precision(1) it reads the activations' high parts alone
-  const uintptr_t base = reinterpret_cast<uintptr_t>(trellis);
-  const int forced = g_prefill_kernel.load();
-  const bool tile = forced != 1 && tile_rate(bits_x2) && (base & 15) == 0 &&
-                    tiles_k * tiles_n * 16 * bits_x2 <= INT_MAX && rows * 4 * kp <= INT_MAX;
+  // the tile GEMM; under exl3_set_tile_precision(1) it reads the
+  // activations' high parts alone
+  const bool tile = tile_applies(trellis, tiles_k, tiles_n, bits_x2, rows);
   const bool tile_lo = !tile_fp16_only();
   const bool lo = !tile || tile_lo;
   {
-    // the register cache sized to the 4-block groups a wavefront forms
-    const int64_t per_wave = ((kp / 128 + 3) / 4 + 3) / 4;
+    // a wavefront per 4-block group of the row, up to 16; the register cache
+    // sized to the groups a wavefront forms
+    const int64_t groups = (kp / 128 + 3) / 4;
     const dim3 grid{unsigned(rows)};
-    if (per_wave <= 1) {
-      hipLaunchKernelGGL(prefill_input<1>, grid, dim3(256), 0, stream, x, x_dtype, logical_in, kp, suh, act, row_exp, lo);
-    } else if (per_wave <= 2) {
-      hipLaunchKernelGGL(prefill_input<2>, grid, dim3(256), 0, stream, x, x_dtype, logical_in, kp, suh, act, row_exp, lo);
+#define VQ_INPUT(C, W)                                                                                        \
+  hipLaunchKernelGGL((prefill_input<C, W>), grid, dim3(64 * W), 0, stream, x, x_dtype, logical_in, kp, suh, act, \
+                     row_exp, lo)
+    if (groups <= 4) {
+      VQ_INPUT(1, 4);
+    } else if (groups <= 8) {
+      VQ_INPUT(1, 8);
+    } else if (groups <= 16) {
+      VQ_INPUT(1, 16);
     } else {
-      hipLaunchKernelGGL(prefill_input<4>, grid, dim3(256), 0, stream, x, x_dtype, logical_in, kp, suh, act, row_exp, lo);
+      VQ_INPUT(2, 16);
     }
+#undef VQ_INPUT
   }
   if (int rc = vq::check_launch("exl3 prefill_input")) return rc;
   if (tile) {
+    TilePlan p = plan_tile(rows, kp, np);
+    if (!tile_lo) p.blocks = kTileBlocks;  // the FP16-only kernels come in one height
+    // fewer splits where the workspace holds fewer
+    const int64_t beyond = workspace_numel - (tile_elements(rows, kp) + 3) / 4 * 4;
+    const int splits = int(std::max<int64_t>(1, std::min<int64_t>(p.splits, beyond / (rows * np))));
     TileArgs t{};
     t.act = reinterpret_cast<const uint8_t*>(act);
     t.act_row_bytes = 4 * kp;
@@ -493,11 +605,18 @@ int prefill_linear(const void* x, int x_dtype, int64_t rows, const uint8_t* trel
     t.out = out;
     t.out_dtype = out_dtype;
     t.logical_out = logical_out;
-    const dim3 grid(unsigned((np + kTileCols - 1) / kTileCols), unsigned((rows + kTileRows - 1) / kTileRows));
-    return launch_tile_gemm(bits_x2, codebook, false, tile_lo, t, grid, stream);
+    t.tile_rows = p.tile_rows;
+    t.partial = splits > 1 ? workspace + (tile_elements(rows, kp) + 3) / 4 * 4 : nullptr;
+    const dim3 grid(unsigned((np + kTileCols - 1) / kTileCols), unsigned(p.row_tiles), unsigned(splits));
+    if (int rc = launch_tile_gemm(bits_x2, codebook, false, tile_lo, p.blocks, t, grid, stream)) return rc;
+    if (splits == 1) return vq::kOk;
+    const int64_t groups = (rows + 3) / 4 * (np / 128);
+    hipLaunchKernelGGL(tile_output, dim3(unsigned(groups)), dim3(256), 0, stream, t.partial, splits, rows,
+                       np, svh, logical_out, out, out_dtype);
+    return vq::check_launch("exl3 tile_output");
   }
   PrefillArgs a{act, row_exp, trellis, svh, out, rows, kp, np, tiles_n, logical_out, out_dtype};
-  const bool aligned = (base & 3) == 0;
+  const bool aligned = (reinterpret_cast<uintptr_t>(trellis) & 3) == 0;
   int rc = vq::kOk;
   bool done = false;
 #define VQ_CASE(B, C)                                        \

@@ -50,9 +50,9 @@ using vq::kFP32;
 
 constexpr int kThreads = 256;
 constexpr int kMaxGemvRows = 8;
-// Calls of up to this many rows run the small-M kernel in chunks of
-// kMaxGemvRows (each chunk streams the matrix once); the prefill GEMM's
-// 256-row tiles only pay off above it.
+// Calls of up to this many rows that the tile GEMM does not take run the
+// small-M kernel in chunks of kMaxGemvRows (each chunk streams the matrix
+// once).
 constexpr int kGemvChunkedRows = 32;
 
 // Per-rate geometry of the small-M kernel.

@@ -102,14 +102,39 @@ __device__ __forceinline__ float u16_act(uint16_t v, int dtype) {
 // high part alone.
 bool tile_fp16_only();
 
-// Large-M (prefill) dense linear, rows > 32 (exl3_gemm.hip).  Arguments as
-// exl3_linear_out's, validated by it; workspace holds rows * padded_in
-// floats (the FP16 high and low activation halves) plus one int32 row
-// exponent per row.
+// How a dense call runs on the tile GEMM (exl3_gemm.hip): the 16-row blocks
+// of a tile (2, 4 or 8), the row tiles and their rows, and the workgroups
+// its K range is split over.
+struct TilePlan {
+  int blocks;
+  int64_t row_tiles;
+  int tile_rows;
+  int splits;
+};
+constexpr int kTileHeight = 8;  // 16-row blocks of a full-height tile
+TilePlan plan_tile(int64_t rows, int64_t kp, int64_t np);
+
+// FP32 elements of the tile GEMM's activations and row exponents for `rows`
+// rows, and with the partial sums of `splits` K splits after them.
+inline int64_t tile_elements(int64_t rows, int64_t kp) { return rows * (kp + 1); }
+inline int64_t tile_elements(int64_t rows, int64_t kp, int64_t np, int splits) {
+  return splits > 1 ? (tile_elements(rows, kp) + 3) / 4 * 4 + splits * rows * np : tile_elements(rows, kp);
+}
+
+// Whether the tile GEMM can take a call: a rate it serves, a 16-byte aligned
+// trellis (LDS-DMA), 32-bit buffer offsets over the matrix and the
+// activations, and no prefill kernel forced (exl3_set_prefill_kernel).
+bool tile_applies(const void* trellis, int64_t tiles_k, int64_t tiles_n, int64_t bits_x2, int64_t rows);
+
+// Many-row dense linear (exl3_gemm.hip).  Arguments as exl3_linear_out's,
+// validated by it; workspace holds at least rows * padded_in floats (the
+// FP16 high and low activation halves) plus one int32 row exponent per row,
+// and what lies beyond takes the partial sums of the planned K splits, as
+// many as fit.
 int prefill_linear(const void* x, int x_dtype, int64_t rows, const uint8_t* trellis,
                    int64_t tiles_k, int64_t tiles_n, const uint16_t* suh, const uint16_t* svh,
                    int bits_x2, int codebook, int64_t logical_in, int64_t logical_out, void* out,
-                   int out_dtype, float* workspace, hipStream_t stream);
+                   int out_dtype, float* workspace, int64_t workspace_numel, hipStream_t stream);
 
 // The finish of exl3_linear_out: out = RN(H128(sum of `splits` partial rows)
 // * svh) for every (row, 128-column block) (exl3_linear.hip).

@@ -209,6 +209,48 @@ int64_t partial_elements(const GemvPlan& p, int64_t rows, int64_t cols) { return
 }  // namespace
 }  // namespace exl3
 
+namespace exl3 {
+namespace {
+
+// Calls of 9 to 32 rows of at least this many inputs run on the tile GEMM
+// where the workspace holds its activations and sums: one pass over the
+// weights in three launches instead of up to four passes in as many (20 rows of
+// a 4096 x 14336 matrix at 3 bits: 49.1 us in chunks, 29.1 on the tile GEMM).
+// Shorter matrices keep the chunks, whose workspace is smaller.
+constexpr int64_t kTileMinInputs = 1024;
+// The fixed scratch that dense callers cut their rows to (8M floats): the
+// size function asks for no more than it on the K splits' account, so the
+// rows that fit it do not change.
+constexpr int64_t kFixedScratch = int64_t(8) << 20;
+
+// Whether a call of at most kGemvChunkedRows rows runs on the tile GEMM: more
+// rows than one small-M launch takes, at the activations' full precision, and
+// a workspace that holds every planned split.
+bool tile_small(int64_t rows, const void* trellis, int64_t tiles_k, int64_t tiles_n, int64_t bits_x2,
+                int64_t workspace_numel) {
+  const int64_t kp = tiles_k * 16, np = tiles_n * 16;
+  return rows > kMaxGemvRows && kp >= kTileMinInputs && !tile_fp16_only() &&
+         tile_applies(trellis, tiles_k, tiles_n, bits_x2, rows) &&
+         workspace_numel >= tile_elements(rows, kp, np, plan_tile(rows, kp, np).splits);
+}
+
+// The floats below which every call of `rows` rows is refused.  The two
+// paths never run in one call, so the larger need is enough.  Small-M (up to
+// 32 rows, in chunks of 8): the K-split partials at the automatic split
+// count (a call whose plan needs more runs in column ranges that fit).
+// Large-M: the FP16 high / low activations (rows * padded_in floats) and one
+// row exponent per row.
+int64_t linear_minimum(int64_t rows, int64_t padded_in, int64_t padded_out) {
+  const int64_t small_rows = std::min<int64_t>(rows, kMaxGemvRows);
+  const GemvPlan plan = plan_gemv(0, 8, padded_in, padded_out, true);
+  const int64_t small = partial_elements(plan, small_rows, padded_out);
+  const int64_t large = rows > kGemvChunkedRows ? tile_elements(rows, padded_in) : 0;
+  return std::max(small, large);
+}
+
+}  // namespace
+}  // namespace exl3
+
 extern "C" int64_t exl3_linear_workspace_size(int64_t max_rows, int64_t padded_in,
                                               int64_t padded_out) {
   if (max_rows < 0) {
@@ -216,16 +258,19 @@ extern "C" int64_t exl3_linear_workspace_size(int64_t max_rows, int64_t padded_i
     return -1;
   }
   if (exl3::check_padded(padded_in) != vq::kOk || exl3::check_padded(padded_out) != vq::kOk) return -1;
-  // The two paths never run in one call, so the larger need is enough.
-  // Small-M (up to 32 rows, in chunks of 8): the K-split partials at the
-  // automatic split count (a call whose plan needs more runs in column
-  // ranges that fit).  Large-M: the FP16 high / low activations (rows *
-  // padded_in floats) and one row exponent per row.
-  const int64_t small_rows = std::min<int64_t>(max_rows, exl3::kMaxGemvRows);
-  const exl3::GemvPlan plan = exl3::plan_gemv(0, 8, padded_in, padded_out, true);
-  const int64_t small = exl3::partial_elements(plan, small_rows, padded_out);
-  const int64_t large = max_rows > exl3::kGemvChunkedRows ? max_rows * (padded_in + 1) : 0;
-  return std::max(small, large);
+  int64_t size = exl3::linear_minimum(max_rows, padded_in, padded_out);
+  // room for the tile GEMM's K splits at every row count up to max_rows
+  // (heights of whole 16-row blocks and max_rows itself bound the others)
+  for (int64_t r = std::min<int64_t>(max_rows, 16); r > exl3::kMaxGemvRows;
+       r = r < max_rows ? std::min(r + 16, max_rows) : 0) {
+    if (r <= exl3::kGemvChunkedRows && padded_in < exl3::kTileMinInputs) continue;
+    const exl3::TilePlan p = exl3::plan_tile(r, padded_in, padded_out);
+    if (p.blocks == exl3::kTileHeight && p.splits == 1) break;  // more rows, more tiles: no splits
+    const int64_t least = exl3::tile_elements(r, padded_in);
+    const int64_t whole = exl3::tile_elements(r, padded_in, padded_out, p.splits);
+    size = std::max(size, std::min(whole, std::max(least, exl3::kFixedScratch)));
+  }
+  return size;
 }
 
 extern "C" int exl3_linear_prefill_rows(void) { return exl3::kGemvChunkedRows; }
@@ -280,7 +325,7 @@ int check_linear(const void* x, int x_dtype, int64_t rows, int64_t x_cols, const
   }
   int64_t ws_bytes = 0;
   if (workspace_numel >= 0) {
-    const int64_t need = exl3_linear_workspace_size(rows, padded_in, padded_out);
+    const int64_t need = linear_minimum(rows, padded_in, padded_out);
     if (workspace_numel < need) return fail("EXL3 linear workspace is too small");
     if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0) {
       return fail("EXL3 linear workspace must be 16-byte aligned");
@@ -306,7 +351,7 @@ int check_linear(const void* x, int x_dtype, int64_t rows, int64_t x_cols, const
   return kOk;
 }
 
-// The small-M path (rows <= 32, chunks of kMaxGemvRows rows) with `partial`
+// The small-M path (chunks of kMaxGemvRows rows) with `partial`
 // holding `partial_numel` floats for the K-split partials.  A chunk whose
 // partials do not fit runs in column ranges (whole 128-column blocks) that
 // do; every range is its own launch on the stream.
@@ -391,11 +436,12 @@ extern "C" int exl3_linear_out(const void* x, int x_dtype, int64_t rows, int64_t
   }
   if (rows == 0) return vq::kOk;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (rows > exl3::kGemvChunkedRows) {
+  if (rows > exl3::kGemvChunkedRows ||
+      exl3::tile_small(rows, trellis, tiles_k, tiles_n, bits_x2, workspace_numel)) {
     return exl3::prefill_linear(x, x_dtype, rows, static_cast<const uint8_t*>(trellis), tiles_k,
                                 tiles_n, static_cast<const uint16_t*>(suh),
                                 static_cast<const uint16_t*>(svh), int(bits_x2), int(codebook),
-                                logical_in, logical_out, out, out_dtype, workspace, s);
+                                logical_in, logical_out, out, out_dtype, workspace, workspace_numel, s);
   }
   return exl3::small_linear(x, x_dtype, rows, static_cast<const uint8_t*>(trellis), tiles_k, tiles_n,
                             static_cast<const uint16_t*>(suh), static_cast<const uint16_t*>(svh),
@@ -470,11 +516,12 @@ extern "C" int exl3_linear_out_scratch(const void* x, int x_dtype, int64_t rows,
   float* scratch = exl3::scratch_address();
   if (!scratch) return vq::kHipFailure;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (rows > exl3::kGemvChunkedRows) {
+  if (rows > exl3::kGemvChunkedRows ||
+      exl3::tile_small(rows, trellis, tiles_k, tiles_n, bits_x2, exl3::kScratchFloats)) {
     return exl3::prefill_linear(x, x_dtype, rows, static_cast<const uint8_t*>(trellis), tiles_k,
                                 tiles_n, static_cast<const uint16_t*>(suh),
                                 static_cast<const uint16_t*>(svh), int(bits_x2), int(codebook),
-                                logical_in, logical_out, out, out_dtype, scratch, s);
+                                logical_in, logical_out, out, out_dtype, scratch, exl3::kScratchFloats, s);
   }
   return exl3::small_linear(x, x_dtype, rows, static_cast<const uint8_t*>(trellis), tiles_k, tiles_n,
                             static_cast<const uint16_t*>(suh), static_cast<const uint16_t*>(svh),

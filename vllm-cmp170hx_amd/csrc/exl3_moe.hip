@@ -1191,7 +1191,7 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
       t.task_group = int(std::min<int64_t>(8, per_xcd));
       const int64_t groups = (per_xcd + t.task_group - 1) / t.task_group;
       const dim3 grid{unsigned(8 * groups * t.task_group * t.col_tiles), 1u, 1u};
-      return exl3::launch_tile_gemm(tile_bits, 2, true, tile_lo, t, grid, s);
+      return exl3::launch_tile_gemm(tile_bits, 2, true, tile_lo, exl3::kTileBlocks, t, grid, s);
     };
     const int want_bits = fixed == 0 ? int(bits_x2) : 0;
     auto gemv = [&](int projection, int64_t kp, int64_t np, int64_t in_off, int64_t out_off) {

@@ -2,8 +2,10 @@
 //
 // C[r][n] = sum_k A[r][k] W[k][n] for a tile of up to 128 rows x 256 output
 // columns, on v_mfma_f32_16x16x32_f16, then the output transform (unscale
-// the row, H128 over each 128-column block, times svh).  Serves the dense
-// linear above 32 rows (exl3_gemm.hip) and the MoE projections of
+// the row, H128 over each 128-column block, times svh).  Where the tiles are
+// too few to fill the chip, the K range is split over workgroups: each then
+// stores the unscaled sums of its inputs, which tile_output (exl3_gemm.hip)
+// adds and transforms.  Serves the dense linear above 8 rows (exl3_gemm.hip) and the MoE projections of
 // prefill-sized calls (exl3_moe.hip: the tile's rows are one expert's routed
 // assignments).
 //
@@ -61,9 +63,9 @@ constexpr int kTileThreads = 64 * kTileWaves;
 constexpr int kTileCols = 64 * kTileWaves;          // 256
 constexpr int kTileRows = 128;
 constexpr int kTileBlocks = kTileRows / 16;         // 16-row blocks
-constexpr int kTileABufs = 3;
-constexpr int kTileRing = 4;
-constexpr int kTileADma = kTileBlocks / kTileWaves;  // 1 KB activation loads per wave and step
+constexpr int kTileABufs = 3;                       // activation buffers
+constexpr int kTileRing = 4;                        // trellis ring slots, and steps per loop iteration
+static_assert(kTileBlocks == kTileHeight, "the plan's full height");
 constexpr int kTileRedStride = kTileCols + 4;       // epilogue row stride (floats)
 
 // The tile GEMM serves every rate: the trellis of one step of a wavefront
@@ -90,6 +92,11 @@ struct TileArgs {
   void* out;
   int out_dtype;
   int64_t logical_out;
+  int tile_rows;           // rows per row tile (a multiple of 16)
+  // dense, K split over gridDim.z workgroups (> 1): FP32 sums of split z's
+  // inputs, unscaled, at partial + z * rows * np; null: the whole K range in
+  // one workgroup, which applies the output transform itself
+  float* partial;
   // MoE: the route table (header, sorted assignments, tasks) and the
   // projection of the experts' tables; FP32 outputs [assignment][np]
   const int* table;
@@ -142,13 +149,30 @@ __device__ __forceinline__ void tile_ready(uint32_t (&w)[2][2][kWords]) {
       for (int i = 0; i < kWords; ++i) asm volatile("" : "+v"(w[p][h][i]));
 }
 
-template <int kBitsX2, int kCodebook, bool kMoe, bool kLo>
-__global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
-  constexpr int kRows = kTileRows;
-  constexpr int kBlocks = kRows / 16;
-  constexpr int kADma = kBlocks / kTileWaves;
+// LDS of a workgroup, and the workgroups a CU holds: as many as the
+// accumulators of `blocks` row blocks leave registers for, and the LDS.
+constexpr int tile_lds_bytes(int blocks, int parts, int bits_x2) {
+  return kTileABufs * parts * blocks * 1024 + kTileWaves * kTileRing * tile_slot_bytes(bits_x2);
+}
+constexpr int tile_occupancy(int blocks, int bits_x2) {
+  const int registers = blocks <= 2 ? 4 : (blocks <= 4 ? 3 : 2);
+  const int lds = 160 * 1024 / tile_lds_bytes(blocks, 2, bits_x2);
+  return registers < lds ? registers : lds;
+}
+
+// kBlocks: the tile's 16-row blocks: 8 (up to 128 rows), or 2 and 4 for dense
+// calls of up to 32 and 64 rows, whose smaller accumulators and activation
+// tiles leave room for more wavefronts per SIMD.  At 2 row blocks a wavefront
+// and step take 0.43 us (900 cycles: the decode's 126 VALU instructions and 16
+// MFMAs, which share the SIMD's issue and add up) whether one or four
+// wavefronts share a SIMD; loads 5 to 8 steps ahead instead of 2 to 4
+// changed nothing.
+template <int kBitsX2, int kCodebook, bool kMoe, bool kLo, int kBlocks>
+__global__ __launch_bounds__(kTileThreads, tile_occupancy(kBlocks, kBitsX2)) void tile_gemm(TileArgs a) {
+  constexpr int kRows = 16 * kBlocks;
   constexpr int kParts = kLo ? 2 : 1;      // activation parts: high (and low)
-  constexpr int kAL = kParts * kADma;      // activation loads per wavefront and step
+  constexpr int kAL = kParts * kBlocks / kTileWaves;  // activation loads per wavefront and step
+  static_assert(kAL >= 1 && kAL * kTileWaves == kParts * kBlocks, "whole activation loads");
   static_assert(tile_rate(kBitsX2), "a rate the tile GEMM serves");
   constexpr int kWords = LaneLoad<kBitsX2>::kWords;
   constexpr int kTileBytes = 16 * kBitsX2;
@@ -157,11 +181,16 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
   constexpr int kTL = kSlot / 1024;          // trellis loads per wavefront and step
   constexpr int kChunkLanes = kRowChunk / 16;
   static_assert(kRowChunk % 16 == 0 && 2 * kRowChunk <= kSlot, "a step's trellis fits its slot");
-  // 80 KB at most (two workgroups per CU in 160 KB)
-  __shared__ __attribute__((aligned(16))) uint8_t a_lds[kTileABufs][kParts * kBlocks][1024];
-  __shared__ __attribute__((aligned(16))) uint8_t t_lds[kTileWaves][kTileRing][kSlot];
-  static_assert(sizeof(a_lds) + sizeof(t_lds) <= 80 * 1024, "two workgroups per CU");
-  static_assert(sizeof(t_lds) >= 2 * kRows * sizeof(int), "the epilogue's row table fits the ring");
+  // the activation buffers, then the wavefronts' trellis rings; the epilogue
+  // keeps 16 rows of sums at its start and the row table at its end
+  constexpr int kABuf = kParts * kBlocks * 1024;
+  constexpr int kAhead = kTileABufs - 1;  // steps the activation loads run ahead
+  static_assert(kTileRing >= kAhead, "the order of the prologue's loads");
+  constexpr int kABytes = kTileABufs * kABuf;
+  constexpr int kTBytes = kTileWaves * kTileRing * kSlot;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kABytes + kTBytes];
+  static_assert(sizeof(lds) == tile_lds_bytes(kBlocks, kParts, kBitsX2), "the LDS the occupancy counts on");
+  static_assert(sizeof(lds) >= 16 * kTileRedStride * sizeof(float) + 2 * kRows * sizeof(int), "the epilogue fits");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -225,8 +254,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
       return;
     }
   } else {
-    const int64_t row0 = int64_t(blockIdx.y) * kRows;
-    nrows = int(a.rows - row0 < kRows ? a.rows - row0 : kRows);
+    const int64_t row0 = int64_t(blockIdx.y) * a.tile_rows;
+    nrows = int(a.rows - row0 < a.tile_rows ? a.rows - row0 : a.tile_rows);
     trellis = a.trellis;
     svh = a.svh;
     tiles_n = a.tiles_n;
@@ -238,7 +267,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
     if constexpr (kMoe) {
       return a.table[4 + first + t];
     } else {
-      return int(int64_t(blockIdx.y) * kRows + t);
+      return int(int64_t(blockIdx.y) * a.tile_rows + t);
     }
   };
   // thread t < kRows keeps row t's id and exponent for the epilogue
@@ -249,7 +278,17 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
   }
 
   const int nblocks = (nrows + 15) >> 4;  // 16-row blocks with rows
-  const int steps = int(a.kp / 32);
+  // this workgroup's K range, in steps of 32 inputs: whole 128-input blocks,
+  // spread evenly over the splits
+  int step0 = 0;
+  int steps = int(a.kp / 32);
+  if constexpr (!kMoe) {
+    const int k_blocks = steps / 4;
+    const int b0 = int(blockIdx.z) * k_blocks / int(gridDim.z);
+    const int b1 = (int(blockIdx.z) + 1) * k_blocks / int(gridDim.z);
+    step0 = 4 * b0;
+    steps = 4 * (b1 - b0);
+  }
   const int last = steps - 1;
   const int row_bytes = int(tiles_n * kTileBytes);
   const int64_t tc0 = col0 / 16 + 4 * wave;  // this wavefront's first tile column
@@ -262,8 +301,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
   // step's two tile rows copy the first chunk again, into the slot's unread
   // tail); chunk c lands at byte 16 c of the slot
   const __amdgpu_buffer_rsrc_t t_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(trellis + tc_load * kTileBytes), 0, (steps * 2 - 1) * row_bytes + kRowChunk,
-      0x00020000);
+      const_cast<uint8_t*>(trellis + tc_load * kTileBytes + int64_t(2 * step0) * row_bytes), 0,
+      (steps * 2 - 1) * row_bytes + kRowChunk, 0x00020000);
   int t_voff[kTL];
 #pragma unroll
   for (int u = 0; u < kTL; ++u) {
@@ -273,54 +312,38 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
   // (each builtin's offsets are locals: an array element passed straight
   // to the builtin makes the host compilation drop the kernel's launch stub)
   auto load_trellis = [&](int s) {
+    const int from = min(s, last);
 #pragma unroll
     for (int u = 0; u < kTL; ++u) {
       const int voff = t_voff[u];
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(t_rsrc, (tile_lds_ptr_t)&t_lds[wave][s % kTileRing][1024 * u], 16,
-                                               voff, s * 2 * row_bytes, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(t_rsrc, (tile_lds_ptr_t)&lds[kABytes + (wave * kTileRing + s % kTileRing) * kSlot + 1024 * u],
+                                               16, voff, from * 2 * row_bytes, 0, 0);
     }
   };
-  // activations: this wavefront's row blocks rb = kADma * wave + i; lane
-  // (g, m) copies group g of row 16 rb + m, its high part into block rb of
-  // the buffer and its low part (2 kp bytes on) into block kBlocks + rb
+  // activations: blocks 0 .. kBlocks - 1 of a buffer are the row blocks'
+  // high parts, the next kBlocks their low parts (2 kp bytes on in the row);
+  // this wavefront copies blocks kAL * wave + i: lane (g, m) group g of row
+  // m of the block
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(a.act), 0, int(a.act_rows * a.act_row_bytes), 0x00020000);
-  const int lo_off = int(2 * a.kp);
-  int a_voff[kADma];
+  int a_voff[kAL];
 #pragma unroll
-  for (int i = 0; i < kADma; ++i) {
-    const int rb = kADma * wave + i;
-    a_voff[i] = int(int64_t(row_of(16 * rb + m)) * a.act_row_bytes + 16 * g);
+  for (int i = 0; i < kAL; ++i) {
+    const int blk = kAL * wave + i;
+    a_voff[i] = int(int64_t(row_of(16 * (blk % kBlocks) + m)) * a.act_row_bytes + 16 * g + 64 * step0) +
+                (blk >= kBlocks ? int(2 * a.kp) : 0);
   }
   auto load_act = [&](int s) {
     const int buf = s % kTileABufs;
+    const int from = min(s, last);
 #pragma unroll
-    for (int i = 0; i < kADma; ++i) {
-      const int hi_voff = a_voff[i];
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (tile_lds_ptr_t)&a_lds[buf][kADma * wave + i][0],
-                                               16, hi_voff, s * 64, 0, 0);
-      if constexpr (kLo) {
-        const int lo_voff = hi_voff + lo_off;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc,
-                                                 (tile_lds_ptr_t)&a_lds[buf][kBlocks + kADma * wave + i][0],
-                                                 16, lo_voff, s * 64, 0, 0);
-      }
+    for (int i = 0; i < kAL; ++i) {
+      const int voff = a_voff[i];
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (tile_lds_ptr_t)&lds[buf * kABuf + (kAL * wave + i) * 1024],
+                                               16, voff, from * 64, 0, 0);
     }
   };
 
-  // ring words: tile column t = 2 p + (m >> 3) of tile row h of the slot
-  int word_off[2][2][kWords];
-  {
-    int idx[kWords];
-    lane_word_index<kBitsX2>(L, idx);
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < kWords; ++i)
-          word_off[p][h][i] = h * kRowChunk + (2 * p + (m >> 3)) * kTileBytes + 4 * idx[i];
-  }
   f32x4_t acc[kBlocks][2][2];
 #pragma unroll
   for (int rb = 0; rb < kBlocks; ++rb)
@@ -330,24 +353,28 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
   // LDS reads in the loop go through tile_read* (outside the compiler's
   // tracking of the LDS-DMA loads, which would make each read wait for
   // every load in flight); tile_ready names the values a wait made ready.
-  const uint32_t a_lane = vq::lds_address(&a_lds[0][0][0]) + 16 * lane;
-  const uint32_t t_base = vq::lds_address(&t_lds[wave][0][0]);
-  uint32_t word_addr[2][2][kWords];
+  const uint32_t a_lane = vq::lds_address(&lds[0]) + 16 * lane;
+  // ring words: tile column t = 2 p + (m >> 3) of tile row h of the slot (p
+  // and h in the read's immediate offset)
+  uint32_t word_addr[kWords];
+  {
+    int idx[kWords];
+    lane_word_index<kBitsX2>(L, idx);
+    const uint32_t t_base = vq::lds_address(&lds[0]) + kABytes + wave * kTileRing * kSlot + (m >> 3) * kTileBytes;
 #pragma unroll
-  for (int p = 0; p < 2; ++p)
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int i = 0; i < kWords; ++i) word_addr[p][h][i] = t_base + word_off[p][h][i];
+    for (int i = 0; i < kWords; ++i) word_addr[i] = t_base + 4 * idx[i];
+  }
   uint32_t words[2][2][kWords];
   auto read_words = [&](auto slot) {
     constexpr int kSlotIdx = decltype(slot)::value;
+    static_for<2>([&](auto p_tag) {
+      static_for<2>([&](auto h_tag) {
+        constexpr int p = decltype(p_tag)::value, h = decltype(h_tag)::value;
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < kWords; ++i) tile_read4<kSlotIdx * kSlot>(words[p][h][i], word_addr[p][h][i]);
+        for (int i = 0; i < kWords; ++i)
+          tile_read4<kSlotIdx * kSlot + h * kRowChunk + 2 * p * kTileBytes>(words[p][h][i], word_addr[i]);
+      });
+    });
   };
 
   // decode of step words w into B operands of pair p: first / second MFMA
@@ -369,16 +396,16 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
     constexpr int kS = decltype(slot)::value;
     constexpr int kRB = decltype(row_blocks)::value;
     static_assert(kRB >= 2, "two row blocks read ahead");
-    load_act(min(s + 2, last));
-    // T(s + 1) landed: after it came A(s), T(s + 2), A(s + 1), T(s + 3),
-    // A(s + 2)
-    vq::wait_vmcnt<3 * kAL + 2 * kTL>();
+    load_act(s + kAhead);
+    // T(s + 1) landed: after it came the activation and trellis loads of the
+    // kTileRing - 2 steps before this one, and this step's activation load
+    vq::wait_vmcnt<(kTileRing - 1) * kAL + (kTileRing - 2) * kTL>();
     read_words(std::integral_constant<int, (kS + 1) % kTileRing>{});  // (past the last step: unused)
-    // this step's slot (its words read and decoded a step ago) takes step s + 4
-    load_trellis(min(s + 4, last));
+    // this step's slot (its words read and decoded a step ago) takes step s + kTileRing
+    load_trellis(s + kTileRing);
 
     half8_t b_next[2][2];
-    const uint32_t a_buf = a_lane + uint32_t(s % kTileABufs) * (kParts * kBlocks * 1024);
+    const uint32_t a_buf = a_lane + uint32_t(s % kTileABufs) * kABuf;
     half8_t ah[kRB], al[kRB];
     auto read_a = [&](auto rb_tag) {
       constexpr int rb = decltype(rb_tag)::value;
@@ -418,17 +445,16 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
       b_cur[p][0] = b_next[p][0];
       b_cur[p][1] = b_next[p][1];
     }
-    // A(s + 1) of this wavefront landed: after it came T(s + 3), A(s + 2),
-    // T(s + 4); then every wavefront's (and every read of buffer s) is done
-    vq::wait_vmcnt<kAL + 2 * kTL>();
+    // A(s + 1) of this wavefront landed: after it came its step's trellis
+    // load and both loads of the kAhead - 1 steps since; then every
+    // wavefront's (and every read of buffer s) is done
+    vq::wait_vmcnt<(kAhead - 1) * kAL + kAhead * kTL>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  // Row blocks past the tile's rows hold copies of its last row: a tile of
-  // up to half the rows runs the half-height loop, any other the full one;
-  // an MoE task (an expert's rows, often well under 128) the loop of its
-  // height rounded up to 2, 4, 5, 6 or 8 row blocks.  None branches around
-  // an MFMA.
+  // Row blocks past the tile's rows hold copies of its last row: a tile
+  // runs the loop of its height rounded up to 2, 4, 5, 6 or 8 row blocks (3
+  // or 4 in a four-block tile).  None branches around an MFMA.
   auto run = [&](auto row_blocks) __attribute__((always_inline)) {
     for (int s = 0; s < steps; s += kTileRing) {
       step(s, std::integral_constant<int, 0>{}, row_blocks);
@@ -437,7 +463,6 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
       step(s + 3, std::integral_constant<int, 3>{}, row_blocks);
     }
   };
-  static_assert(kBlocks == 8, "row-block heights below");
   // A wavefront whose tile columns all lie past the matrix (in the last
   // column tile of a projection whose width is no multiple of 256) only
   // loads its share of the activation tiles and meets every barrier: its
@@ -445,27 +470,27 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
   const bool idle = tc0 >= tiles_n;
   if (idle) {
     asm volatile("" ::: "memory");
-    load_act(0);
-    load_act(min(1, last));
-    vq::wait_vmcnt<kAL>();  // A(0) of this wavefront landed
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) load_act(i);
+    vq::wait_vmcnt<(kAhead - 1) * kAL>();  // A(0) of this wavefront landed
     __builtin_amdgcn_s_barrier();
     for (int s = 0; s < steps; ++s) {
       asm volatile("" ::: "memory");
-      load_act(min(s + 2, last));
-      vq::wait_vmcnt<kAL>();  // A(s + 1) of this wavefront landed
+      load_act(s + kAhead);
+      vq::wait_vmcnt<(kAhead - 1) * kAL>();  // A(s + 1) of this wavefront landed
       __builtin_amdgcn_s_barrier();
     }
     asm volatile("" ::: "memory");
   } else {
-    // ---- prologue: T(0), T(1), A(0), T(2), A(1), T(3) in that order ----
+    // ---- prologue: the loads of the kTileRing steps before step 0, in the
+    // order those steps would issue them (each A before its step's T) ----
     asm volatile("" ::: "memory");
-    load_trellis(0);
-    load_trellis(min(1, last));
-    load_act(0);
-    load_trellis(min(2, last));
-    load_act(min(1, last));
-    load_trellis(min(3, last));
-    vq::wait_vmcnt<kAL + 2 * kTL>();  // T(0), T(1) and A(0) of this wavefront landed
+#pragma unroll
+    for (int i = 0; i < kTileRing; ++i) {
+      if (i >= kTileRing - kAhead) load_act(i - (kTileRing - kAhead));
+      load_trellis(i);
+    }
+    vq::wait_vmcnt<(kAhead - 1) * kAL + kAhead * kTL>();  // A(0) and every load before it landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read_words(std::integral_constant<int, 0>{});
@@ -473,7 +498,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
     tile_ready(words);
     decode_pair(words, 0, b_cur);
     decode_pair(words, 1, b_cur);
-    if constexpr (kMoe) {
+    if constexpr (kBlocks == 8) {
       if (nblocks > 6) {
         run(std::integral_constant<int, 8>{});
       } else if (nblocks > 5) {
@@ -485,10 +510,14 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
       } else {
         run(std::integral_constant<int, 2>{});
       }
-    } else if (nblocks > kBlocks / 2) {
-      run(std::integral_constant<int, kBlocks>{});
+    } else if constexpr (kBlocks == 4) {
+      if (nblocks > 3) {
+        run(std::integral_constant<int, 4>{});
+      } else {
+        run(std::integral_constant<int, 3>{});
+      }
     } else {
-      run(std::integral_constant<int, kBlocks / 2>{});
+      run(std::integral_constant<int, kBlocks>{});
     }
   }
 
@@ -497,7 +526,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
   // the epilogue reuses
   vq::wait_vmcnt<0>();
   __syncthreads();
-  int* row_id = reinterpret_cast<int*>(&t_lds[0][0][0]);
+  int* row_id = reinterpret_cast<int*>(&lds[kABytes + kTBytes - 2 * kRows * sizeof(int)]);
   int* row_e = row_id + kRows;
   if (tid < kRows) {
     row_id[tid] = my_row;
@@ -518,8 +547,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
   float sv[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) sv[j] = c0 + j < a.np ? vq::f16_to_f32(svh[c0 + j]) : 0.0f;
-  float* red = reinterpret_cast<float*>(&a_lds[0][0][0]);  // [16][kTileRedStride]
-  static_assert(sizeof(a_lds) >= 16 * kTileRedStride * sizeof(float), "epilogue rows fit");
+  float* red = reinterpret_cast<float*>(&lds[0]);  // [16][kTileRedStride]
 #pragma unroll
   for (int rb = 0; rb < kBlocks; ++rb) {
     // (row blocks past the tile's rows store nothing: the workgroup stops
@@ -553,6 +581,16 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
         v[j] = y0;
         v[4 + j] = y1;
       }
+      if constexpr (!kMoe) {
+        if (a.partial) {
+          // a split's sums: the output transform follows once they are added
+          if (tr < nrows) {
+            const int64_t row = int64_t(blockIdx.z) * a.rows + int64_t(blockIdx.y) * a.tile_rows + tr;
+            vq::store8_act(a.partial, vq::kFP32, row * a.np + c0, v, a.np - c0);
+          }
+          continue;
+        }
+      }
       vq::h128_rows(v, l);
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] *= sv[j];
@@ -560,7 +598,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
         if constexpr (kMoe) {
           vq::store8_act(a.moe_out, vq::kFP32, int64_t(row_id[tr]) * a.np + c0, v, a.np - c0);
         } else {
-          const int64_t row = int64_t(blockIdx.y) * kRows + tr;
+          const int64_t row = int64_t(blockIdx.y) * a.tile_rows + tr;
           vq::store8_act(a.out, a.out_dtype, row * a.logical_out + c0, v, a.logical_out - c0);
         }
       }
@@ -575,15 +613,16 @@ __global__ __launch_bounds__(kTileThreads, 2) void tile_gemm(TileArgs a) {
 // mul1 rates, its MoE kernels.
 constexpr int kTileParts = 4;
 
-// Launches tile_gemm<bits_x2, codebook, moe, lo> for a format of part P
-// (a format of another part is refused).
+// Launches tile_gemm<bits_x2, codebook, moe, lo, blocks> for a format of
+// part P (a format of another part is refused).  blocks: 8, or 2 or 4 for
+// dense calls on high and low parts.
 template <int P>
-int tile_launch_part(int64_t bits_x2, int64_t codebook, bool moe, bool lo, const TileArgs& a, dim3 grid,
-                     hipStream_t stream);
+int tile_launch_part(int64_t bits_x2, int64_t codebook, bool moe, bool lo, int blocks, const TileArgs& a,
+                     dim3 grid, hipStream_t stream);
 
-// Launches tile_gemm<bits_x2, codebook, moe, lo> from the part that holds it
-// (exl3_gemm.hip).
-int launch_tile_gemm(int64_t bits_x2, int64_t codebook, bool moe, bool lo, const TileArgs& a, dim3 grid,
-                     hipStream_t stream);
+// Launches tile_gemm<bits_x2, codebook, moe, lo, blocks> from the part that
+// holds it (exl3_gemm.hip).
+int launch_tile_gemm(int64_t bits_x2, int64_t codebook, bool moe, bool lo, int blocks, const TileArgs& a,
+                     dim3 grid, hipStream_t stream);
 
 }  // namespace exl3
