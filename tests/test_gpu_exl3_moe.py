@@ -573,3 +573,27 @@ def test_moe_rejects_bad_arguments(ops, device):
         ops.moe_out(x, ids[:1], weights[:1], layer.ptrs, layer.meta, emap, intermediate, out, ws)
     with pytest.raises(RuntimeError, match="mul1"):
         ops.moe_out_v2(x, ids, weights, layer.ptrs, layer.meta, emap, intermediate, 9, out, ws)
+
+
+def test_moe_out_every_rate_in_one_layer_matches_oracle(ops, device):
+    """moe_out's mixed kernel: one layer whose matrices take every mul1 rate
+    (each its specialized loop) and mcg (run-time decode), with expert row
+    counts around the 8-row sub-blocks and the 32-row tasks."""
+    print("moe_out every rate", flush=True)
+    rng = np.random.default_rng(321)
+    hidden, intermediate = 384, 256
+    formats = [(b, 2) for b in (2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16)] + [(4, 1), (10, 1)]
+    counts = [1, 7, 8, 9, 15, 16, 17, 24, 31, 32, 33, 64, 70]
+    experts = len(formats)
+    layer = Layer(rng, experts, hidden, intermediate, formats, device)
+    # one slot a row: expert e is routed counts[e] rows, in a shuffled order
+    flat = rng.permutation(np.repeat(np.arange(experts), counts)).astype(np.int32)
+    rows = flat.size
+    x, code, xt = _acts(rng, rows, hidden, "bf16", device)
+    ids = flat.reshape(rows, 1)
+    weights = rng.random((rows, 1)).astype(np.float32) + 0.5
+    expert_map = np.arange(experts, dtype=np.int64)
+    got = _run(ops, xt, _dev(ids, device), _dev(weights, device), layer, _dev(expert_map, device),
+               intermediate)
+    want = O.moe_out(x, code, ids, weights, layer.oracle, expert_map, intermediate)
+    _assert_moe_close(_out_np(got), _oracle_f32(want, code), "every rate")

@@ -5,8 +5,7 @@
 // Launch sequence on the caller's stream (as the reference's run_moe_out):
 //  1. moe_route groups the local assignments by local expert (counts,
 //     scan, sorted list: the GEMV experts' rows, then the tile experts'
-//     rows) and cuts each expert's rows into tasks of at most 32 rows (8 for
-//     the run-time-format decode: the per-expert token sort): one workgroup
+//     rows) and cuts each expert's rows into tasks of at most 32 rows: one workgroup
 //     below 8192 routed slots, else moe_route_count / moe_route /
 //     moe_route_fill over many workgroups.
 //  2. per projection (gate, up): moe_form builds t = H128(x[a / topk] * suh)
@@ -30,9 +29,10 @@
 //  5. moe_combine: per token, one FMA per local route in route order with
 //     the routing weight, rounded to the output dtype.
 //
-// Expert formats come from packed_meta on the device.  moe_out decodes any
-// admitted format at run time; moe_out_v2 (one bits_x2 for the layer, mul1)
-// runs the decode specialized for that rate.
+// Expert formats come from packed_meta on the device.  moe_out takes any
+// admitted format per matrix (each task the decode specialized for its mul1
+// rate; mcg at run time); moe_out_v2 (one bits_x2 for the layer, mul1) runs
+// the kernel built for that rate.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -52,17 +52,9 @@ namespace {
 constexpr int kRouteThreads = 1024;
 constexpr int64_t kMaxRouteExperts = 4096;
 // Rows of one expert per GEMV task: every decoded weight operand feeds the
-// MFMAs of up to four 8-row sub-blocks, so a fixed-rate expert's weights
-// are decoded once per 32 of its rows.  The run-time-format decode needs the
-// registers the extra accumulators would take: 8 rows there.
+// MFMAs of up to four 8-row sub-blocks, so an expert's weights are decoded
+// once per 32 of its rows.
 constexpr int kTaskRows = 32;
-constexpr int task_rows(int bits_x2) { return bits_x2 > 0 ? kTaskRows : 8; }
-// The rate of the fixed-rate GEMV serving a call's bits_x2 (moe_out_v2's
-// mul1 rates 2..16 and moe_out_prefill's 10, decoded by specialized
-// kernels), or 0: the run-time-format decode, which serves moe_out (any
-// admitted format per expert).
-constexpr int fixed_rate(int64_t bits_x2) { return bits_x2 >= 2 && bits_x2 <= 16 ? int(bits_x2) : 0; }
-
 // Routing of one call (reference: csrc/exl3/moe.cu:19-55).
 struct Routing {
   const void* ids;          // [rows][topk] int32 or int64 global expert ids
@@ -678,37 +670,63 @@ __device__ __forceinline__ void progress_priority(int step, int steps) {
   }
 }
 
+// A GEMV launch: gridDim.z projections from `projection` on, projection +
+// z reading the B operands at in_offset + z * in_step (floats of the
+// workspace) and the row exponents in slot z of each assignment, and writing
+// its rows at out_offset + z * out_step.
+struct MoeGemvArgs {
+  int projection;
+  int64_t kp;
+  int64_t np;
+  const int* table;
+  float* ws;
+  int64_t in_offset, in_step;
+  int64_t out_offset, out_step;
+};
+
+// LDS of a workgroup: two buffers of one 128-input block's B operands,
+// [buf][step][g][column][8 halves] (the epilogue's per-row sums reuse them:
+// kTaskRows x 128 floats), and the rows' exponents.
+constexpr int kTaskCols = 2 * kTaskRows;
+struct MoeGemvShared {
+  _Float16 bop[2][4][4][kTaskCols][8];
+  int rexp[kTaskRows];
+};
+static_assert(sizeof(MoeGemvShared::bop) >= sizeof(float) * kTaskRows * 128, "row sums fit the B staging");
+
 // One workgroup = (task, 128 output columns); wavefront w owns the column
 // pair (two tile columns) 4 * blockIdx.x + w over the whole K range.  Each
 // decoded step (two tile rows, 16 weights a lane) is an A operand of the
 // MFMAs of every 8-row sub-block of the task (B columns 2r, 2r + 1: row r's
 // high and low parts); the sums run over the whole row (one scale per
 // assignment row) and fold once.
-// kBitsX2 = 0: the expert's format at run time.
-// want_bits (run-time decode only): the layer's mul1 rate every expert must
-// have (moe_out_v2 above 4 bits), or 0 for any admitted format (moe_out).
-template <int kBitsX2>
-__global__ __launch_bounds__(256, kBitsX2 > 8 ? 3 : (kBitsX2 > 0 ? 4 : 2)) void moe_gemv(Routing routing, int projection, int64_t kp,
-                                                int64_t np, const int* table, float* ws,
-                                                MoeLayout lay, int64_t in_offset,
-                                                int64_t out_offset, int want_bits) {
+// kBitsX2 = 0: the expert's format at run time (kAnyBase: the decode reads
+// the tiles itself); else mul1 at that rate, kAnyBase also on trellises at
+// 2-byte offsets.
+template <int kBitsX2, bool kAnyBase>
+__device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeGemvArgs& args, const MoeLayout& lay,
+                                              MoeGemvShared& shared) {
   constexpr bool kFixed = kBitsX2 > 0;
   // steps of trellis loads in flight: one B block, so the loop body below
   // is one block with no branch around a load (steps is a multiple of 4)
   constexpr int kDepth = 4;
-  constexpr int kRows = task_rows(kBitsX2);
+  constexpr int kRows = kTaskRows;
   constexpr int kSub = kRows / 8;
-  constexpr int kCols = 2 * kRows;
+  constexpr int kCols = kTaskCols;
   constexpr int kChunks = kCols / 16;  // 16-byte B chunks per thread per block
-  // one 128-input block of B operands: [buf][step][g][column][8 halves]
-  // (the epilogue's per-row sums reuse it: kRows x 128 floats)
-  __shared__ __attribute__((aligned(16))) _Float16 bop[2][4][4][kCols][8];
-  __shared__ int rexp[kRows];
-  static_assert(sizeof(bop) >= sizeof(float) * kRows * 128, "row sums fit the B staging");
+  auto& bop = shared.bop;
+  auto& rexp = shared.rexp;
   float (*red)[128] = reinterpret_cast<float (*)[128]>(&bop[0][0][0][0][0]);
 
+  const int z = int(blockIdx.z);
+  const int projection = args.projection + z;
+  const int64_t kp = args.kp;
+  const int64_t np = args.np;
+  const int* table = args.table;
+  float* ws = args.ws;
+  const int64_t in_offset = args.in_offset + z * args.in_step;
+  const int64_t out_offset = args.out_offset + z * args.out_step;
   const int64_t task = blockIdx.y;
-  if (task >= table[1]) return;
   // the task, the expert's pointers and geometry are read with vector loads
   // (the table lies in the workspace this kernel writes): uniform() keeps
   // them, and the buffer resources built from them, in scalar registers
@@ -738,10 +756,9 @@ __global__ __launch_bounds__(256, kBitsX2 > 8 ? 3 : (kBitsX2 > 0 ? 4 : 2)) void 
   // admitted format) would be read out of bounds: its rows get NaN instead.
   const bool bad = meta[0] != kp || meta[1] != np ||
                    (kFixed ? (meta[2] != kBitsX2 || meta[3] != 2)
-                           : (want_bits > 0 && (meta[2] != want_bits || meta[3] != 2)) ||
-                                 !(meta[3] == 1 ? (bits_x2 >= 2 && bits_x2 <= 16 && bits_x2 % 2 == 0)
-                                                : (meta[3] == 2 && bits_x2 >= 2 && bits_x2 <= 16 &&
-                                                   (bits_x2 % 2 == 0 || bits_x2 <= 7))));
+                           : !(meta[3] == 1 ? (bits_x2 >= 2 && bits_x2 <= 16 && bits_x2 % 2 == 0)
+                                            : (meta[3] == 2 && bits_x2 >= 2 && bits_x2 <= 16 &&
+                                               (bits_x2 % 2 == 0 || bits_x2 <= 7))));
   if (bad) {
     for (int r = wave; r < nrows; r += 4) {
       float* dst = ws + out_offset + int64_t(table[4 + first + r]) * np + 128 * int64_t(blockIdx.x);
@@ -797,7 +814,7 @@ __global__ __launch_bounds__(256, kBitsX2 > 8 ? 3 : (kBitsX2 > 0 ? 4 : 2)) void 
   };
   if (tid < kRows) {
     const int* exps = reinterpret_cast<const int*>(ws + lay.ints()) + lay.exps();
-    rexp[tid] = exps[int64_t(sorted[first + min(tid, nrows - 1)]) * (lay.kmax() / 128)];
+    rexp[tid] = exps[int64_t(sorted[first + min(tid, nrows - 1)]) * (lay.kmax() / 128) + z];
   }
 
   // trellis ring (fixed rate up to 4 bits per weight: one coalesced dword
@@ -939,7 +956,7 @@ __global__ __launch_bounds__(256, kBitsX2 > 8 ? 3 : (kBitsX2 > 0 ? 4 : 2)) void 
     }
   };
   if constexpr (kFixed) {
-    if (aligned) {
+    if (!kAnyBase || aligned) {
       run(std::true_type{});
     } else {
       run(std::false_type{});
@@ -992,6 +1009,38 @@ __global__ __launch_bounds__(256, kBitsX2 > 8 ? 3 : (kBitsX2 > 0 ? 4 : 2)) void 
       dst[c0] = v0 * svh0;
       dst[c0 + 64] = v1 * svh1;
     }
+  }
+}
+
+// A layer of one mul1 rate (moe_out_v2, moe_out_prefill).
+template <int kBitsX2>
+__global__ __launch_bounds__(256, kBitsX2 > 8 ? 3 : 4) void moe_gemv(Routing routing, MoeGemvArgs args, MoeLayout lay) {
+  __shared__ __attribute__((aligned(16))) MoeGemvShared shared;
+  if (blockIdx.y >= args.table[1]) return;
+  moe_gemv_task<kBitsX2, true>(routing, args, lay, shared);
+}
+
+// A layer whose matrices have rates of their own (moe_out): every workgroup
+// takes the loop specialized for its expert's rate (mul1, 4-byte aligned
+// trellis); mcg and other bases are decoded by run-time arithmetic.  Run-time
+// arithmetic for every expert, in tasks of 8 rows and with no trellis load
+// ahead of its use, took 203 us a projection where this takes about 45 (64
+// experts of 2048 / 768 at 3 and 4 bits, 1600 routed rows: 635 -> 172 us a
+// call, bitwise equal).
+__global__ __launch_bounds__(256, 3) void moe_gemv_mixed(Routing routing, MoeGemvArgs args, MoeLayout lay) {
+  __shared__ __attribute__((aligned(16))) MoeGemvShared shared;
+  if (blockIdx.y >= args.table[1]) return;
+  const int expert = vq::uniform(reinterpret_cast<const int4*>(args.table + lay.tasks())[blockIdx.y].x);
+  const int at = expert * 3 + args.projection + int(blockIdx.z);
+  const int64_t trellis = vq::uniform(routing.ptrs[int64_t(at) * 3]);
+  const int64_t bits_x2 = vq::uniform(routing.meta[int64_t(at) * 4 + 2]);
+  const int64_t codebook = vq::uniform(routing.meta[int64_t(at) * 4 + 3]);
+  switch (codebook == 2 && (trellis & 3) == 0 ? bits_x2 : 0) {
+#define VQ_MOE(B) case B: return moe_gemv_task<B, false>(routing, args, lay, shared);
+    VQ_MOE(2) VQ_MOE(3) VQ_MOE(4) VQ_MOE(5) VQ_MOE(6) VQ_MOE(7) VQ_MOE(8)
+    VQ_MOE(10) VQ_MOE(12) VQ_MOE(14) VQ_MOE(16)
+#undef VQ_MOE
+    default: return moe_gemv_task<0, true>(routing, args, lay, shared);
   }
 }
 
@@ -1115,8 +1164,7 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
                         local_experts, topk, ids64 != 0, map64 != 0};
   const bool any = local_experts > 0 && assignments > 0;
   // every check before the first launch
-  const int fixed = exl3::fixed_rate(bits_x2);
-  const int task_rows = exl3::task_rows(fixed);
+  const int task_rows = exl3::kTaskRows;
   const int64_t max_tasks =
       std::min<int64_t>(assignments, (assignments + task_rows - 1) / task_rows + local_experts);
   // Experts with enough rows run on the tile GEMM (a call with one rate for
@@ -1193,17 +1241,16 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
       const dim3 grid{unsigned(8 * groups * t.task_group * t.col_tiles), 1u, 1u};
       return exl3::launch_tile_gemm(tile_bits, 2, true, tile_lo, exl3::kTileBlocks, t, grid, s);
     };
-    const int want_bits = fixed == 0 ? int(bits_x2) : 0;
-    auto gemv = [&](int projection, int64_t kp, int64_t np, int64_t in_off, int64_t out_off) {
-      const dim3 grid(unsigned(np / 128), unsigned(max_tasks));
-      switch (fixed) {
-#define VQ_MOE(B) case B: hipLaunchKernelGGL(exl3::moe_gemv<B>, grid, dim3(256), 0, s, routing, projection, kp, np, table, workspace, lay, in_off, out_off, 0); break;
+    auto gemv = [&](int projection, int projections, int64_t kp, int64_t np, int64_t in_off, int64_t in_step,
+                    int64_t out_off, int64_t out_step) {
+      const dim3 grid(unsigned(np / 128), unsigned(max_tasks), unsigned(projections));
+      const exl3::MoeGemvArgs args{projection, kp, np, table, workspace, in_off, in_step, out_off, out_step};
+      switch (int(bits_x2)) {
+#define VQ_MOE(B) case B: hipLaunchKernelGGL(exl3::moe_gemv<B>, grid, dim3(256), 0, s, routing, args, lay); break;
         VQ_MOE(2) VQ_MOE(3) VQ_MOE(4) VQ_MOE(5) VQ_MOE(6) VQ_MOE(7) VQ_MOE(8)
         VQ_MOE(10) VQ_MOE(12) VQ_MOE(14) VQ_MOE(16)
 #undef VQ_MOE
-        default:
-          hipLaunchKernelGGL(exl3::moe_gemv<0>, grid, dim3(256), 0, s, routing, projection, kp, np,
-                             table, workspace, lay, in_off, out_off, want_bits);
+        default: hipLaunchKernelGGL(exl3::moe_gemv_mixed, grid, dim3(256), 0, s, routing, args, lay);
       }
       return check_launch("exl3 moe_gemv");
     };
@@ -1244,13 +1291,13 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
     for (int p = 0; p < 2; ++p) {
       if (int rc = form(false, p)) return rc;
       const int64_t out_off = p == 0 ? lay.gate() : lay.up();
-      if (int rc = gemv(p, lay.hpad, lay.ipad, lay.input(), out_off)) return rc;
+      if (int rc = gemv(p, 1, lay.hpad, lay.ipad, lay.input(), 0, out_off, 0)) return rc;
       if (tiles) {
         if (int rc = tile(p, lay.hpad, lay.ipad, lay.input(), out_off)) return rc;
       }
     }
     if (int rc = form(true, 2)) return rc;
-    if (int rc = gemv(2, lay.ipad, lay.hpad, lay.act(), lay.input())) return rc;
+    if (int rc = gemv(2, 1, lay.ipad, lay.hpad, lay.act(), 0, lay.input(), 0)) return rc;
     if (tiles) {
       if (int rc = tile(2, lay.ipad, lay.hpad, lay.act(), lay.input())) return rc;
     }
