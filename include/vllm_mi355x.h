@@ -136,12 +136,15 @@ int exl3_linear_out(const void* x, int x_dtype, int64_t rows, int64_t x_cols,
                     float* workspace, int64_t workspace_numel, void* stream);
 
 /*
- * FP32 workspace elements exl3_moe_out needs: with A = max_rows * topk,
+ * FP32 workspace elements exl3_moe_out uses: with A = max_rows * topk,
  * hpad / ipad the hidden / intermediate sizes rounded up to 128,
  * A * (hpad + 3 * ipad) (activations, gate, up and down-input rows) plus the int32
  * routing table (4 + A rounded up to 4 + 4 A) plus A * max(hpad, ipad) / 128
- * int32 scale exponents plus A int32 experts of the sorted rows; 0 when
- * local_experts is 0; -1 (with an error
+ * int32 scale exponents plus A int32 experts of the sorted rows; from hpad
+ * 1024 on, also room for calls of fewer than 8192 slots to form gate and up
+ * together (the larger of the above and, with A at most 8191, the above
+ * rounded up to 4 plus A * hpad).  exl3_moe_out accepts less, down to the
+ * formula without that room.  0 when local_experts is 0; -1 (with an error
  * message) for negative counts or nonpositive sizes.
  * Replaces _exl3_C::moe_workspace_size and moe_workspace_size_v2
  * (csrc/exl3/moe.cu:304-317, csrc/exl3/moe_v2.cu:2041-2061).

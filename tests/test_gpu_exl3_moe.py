@@ -597,3 +597,37 @@ def test_moe_out_every_rate_in_one_layer_matches_oracle(ops, device):
                intermediate)
     want = O.moe_out(x, code, ids, weights, layer.oracle, expert_map, intermediate)
     _assert_moe_close(_out_np(got), _oracle_f32(want, code), "every rate")
+
+
+@pytest.mark.parametrize("rows", [1, 3, 40])
+@pytest.mark.parametrize("path", ["gemv", "tile"])
+def test_moe_gate_and_up_together_equal_one_after_the_other(ops, device, tile_rows, path, rows):
+    """With the sized workspace gate and up are formed and run in one launch
+    each; the smallest workspace accepted (the formula of smaller hidden sizes)
+    runs them one after the other: the same operations, so bitwise equal,
+    and equal to the oracle at the bar."""
+    print(f"moe pair path={path} rows={rows}", flush=True)
+    rng = np.random.default_rng(70 + rows)
+    hidden, intermediate, experts, topk, bits_x2 = 1152, 256, 5, 2, 6
+    tile_rows(1 if path == "tile" else 1 << 20)
+    layer = Layer(rng, experts, hidden, intermediate, [(bits_x2, 2)], device)
+    ids = np.stack([rng.permutation(experts)[:topk] for _ in range(rows)])
+    weights = rng.random((rows, topk)).astype(np.float32)
+    expert_map = np.arange(experts, dtype=np.int64)
+    x_host, code, x = _acts(rng, rows, hidden, "fp16", device)
+    a = rows * topk
+    least = a * (hidden + 3 * intermediate) + 4 + (a + 3) // 4 * 4 + 4 * a + a * hidden // 128 + a
+    sized = ops.moe_workspace_size_v2(rows, hidden, intermediate, topk, experts)
+    assert sized >= least + a * hidden
+    outs = []
+    for size in (sized, least):
+        ws = torch.full((size + 64,), float("nan"), dtype=torch.float32, device=device)
+        out = torch.full_like(x, float("nan"))
+        ops.moe_out_v2(x, _dev(ids, device), _dev(weights, device), layer.ptrs, layer.meta,
+                       _dev(expert_map, device), intermediate, bits_x2, out, ws[:size])
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(ws[size:]).all())
+        outs.append(out)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    want = O.moe_out(x_host, code, ids, weights, layer.oracle, expert_map, intermediate, out_dtype=code)
+    _assert_moe_close(_out_np(outs[0]), _oracle_f32(want, code), f"pair rows={rows}")

@@ -98,7 +98,23 @@ struct MoeLayout {
   __host__ __device__ int64_t exps() const { return tasks() + 4 * assignments; }
   __host__ __device__ int64_t row_experts() const { return exps() + assignments * (kmax() / 128); }
   __host__ __device__ int64_t total() const { return ints() + row_experts() + assignments; }
+  // Where the workspace holds it, the up projection's B operands (A x hpad) in
+  // a region of their own: gate and up are then formed in one launch and run
+  // in one launch, the up rows' exponents in slot 1 of each assignment's
+  // kmax / 128 (so inputs of at least two 128-blocks).
+  __host__ __device__ int64_t input_up() const { return (total() + 3) / 4 * 4; }
+  __host__ __device__ int64_t total_up() const { return input_up() + assignments * hpad; }
 };
+// Calls sized for gate and up together: at least this hidden size (shorter
+// rows' projections are launch-bound either way), and fewer routed slots than
+// kPairMaxSlots.  Few tasks leave a projection's launch short of workgroups
+// (27 slots of a 7168 / 2048 layer: 240 for gate, 88 us each; both together
+// take about 100): 208 -> 150 us a call there, 542 -> 519 at 576 slots.  Many
+// rows' operands for both projections no longer fit the 256 MB last-level cache
+// between their forming and their use: 20480 slots of 2560 / 640 took 881 us one
+// after the other and 903 together.
+constexpr int64_t kPairMinHidden = 1024;
+constexpr int64_t kPairMaxSlots = 8192;
 
 // ---- 1. route ------------------------------------------------------------------
 
@@ -449,7 +465,8 @@ __device__ __forceinline__ void store8(__amdgpu_buffer_rsrc_t dst, int kp, int k
 // group indices), for the row maximum of |t|, then writes the high / low
 // parts at the row's one power-of-two scale, so the expert GEMV sums the
 // whole row before it unscales; groups past the register cache are formed
-// again (the same operations, so the same values).  kWaveRow: each
+// again (the same operations, so the same values).  gridDim.y projections
+// from first_projection on.  kWaveRow: each
 // wavefront forms a sorted row of its own (four rows a workgroup: rows of
 // up to 4 kCache groups, whose chains of dependent loads then overlap four
 // times as deep); otherwise one workgroup a row, wavefront w taking groups
@@ -463,10 +480,12 @@ constexpr int64_t kFormRowGroupsActivate = 2;
 constexpr int64_t kFormRowMin = 8192;
 template <bool kActivate, int kCache, bool kWaveRow>
 __global__ __launch_bounds__(256) void moe_form(Routing routing, const void* x, int x_dtype,
-                                                int64_t hidden, int64_t intermediate, int projection,
+                                                int64_t hidden, int64_t intermediate, int first_projection,
                                                 const int* table, float* ws, MoeLayout lay,
                                                 float limit, bool tile_lo) {
   __shared__ uint32_t row_max;
+  const int z = int(blockIdx.y);  // gate and up in one launch: 0, 1
+  const int projection = first_projection + z;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int q = lane >> 4;   // the lane's block within a group
@@ -487,9 +506,9 @@ __global__ __launch_bounds__(256) void moe_form(Routing routing, const void* x, 
   // at FP16 precision
   const bool lo = tile_lo || table[2] == 0 ||
                   row < reinterpret_cast<const int4*>(table + lay.tasks())[table[3]].y;
-  int* exps = reinterpret_cast<int*>(ws + lay.ints()) + lay.exps() + a * (lay.kmax() / 128);
+  int* exps = reinterpret_cast<int*>(ws + lay.ints()) + lay.exps() + a * (lay.kmax() / 128) + z;
   const __amdgpu_buffer_rsrc_t dst =
-      make_rsrc(ws + (kActivate ? lay.act() : lay.input()) + a * kp, uint32_t(kp) * 4u);
+      make_rsrc(ws + (kActivate ? lay.act() : (z ? lay.input_up() : lay.input())) + a * kp, uint32_t(kp) * 4u);
   const bool bad = routing.meta[e * 12 + projection * 4] != kp;
   const uint16_t* suh = reinterpret_cast<const uint16_t*>(ptrs[projection * 3 + 1]);
   // Buffer resources over the row's inputs (32-bit offsets; loads past the
@@ -1119,7 +1138,10 @@ extern "C" int64_t exl3_moe_workspace_size(int64_t max_rows, int64_t hidden_size
   if (local_experts == 0) return 0;
   const exl3::MoeLayout lay{exl3::padded(hidden_size), exl3::padded(intermediate_size),
                             max_rows * topk};
-  return lay.total();
+  if (lay.hpad < exl3::kPairMinHidden) return lay.total();
+  // (larger calls' workspaces hold any smaller call's pair too)
+  const exl3::MoeLayout pair{lay.hpad, lay.ipad, std::min(lay.assignments, exl3::kPairMaxSlots - 1)};
+  return std::max(lay.total(), pair.total_up());
 }
 
 extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hidden,
@@ -1151,15 +1173,15 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
   if (exl3::padded(hidden) * exl3::padded(intermediate_size) * 2 > INT_MAX) {
     return fail("EXL3 MoE: an expert matrix must stay below 2 GiB");
   }
-  const int64_t need = exl3_moe_workspace_size(rows, hidden, intermediate_size, topk, local_experts);
-  if (need < 0) return kInvalidArgument;
-  if (workspace_numel < need) return fail("EXL3 MoE workspace is too small");
+  const int64_t sized = exl3_moe_workspace_size(rows, hidden, intermediate_size, topk, local_experts);
+  if (sized < 0) return kInvalidArgument;
+  const exl3::MoeLayout lay{exl3::padded(hidden), exl3::padded(intermediate_size), assignments};
+  if (workspace_numel < (local_experts == 0 ? 0 : lay.total())) return fail("EXL3 MoE workspace is too small");
   if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0) {
     return fail("EXL3 MoE workspace must be 16-byte aligned");
   }
   if (rows == 0) return kOk;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const exl3::MoeLayout lay{exl3::padded(hidden), exl3::padded(intermediate_size), assignments};
   exl3::Routing routing{topk_ids, expert_map, packed_ptrs, packed_meta, global_experts,
                         local_experts, topk, ids64 != 0, map64 != 0};
   const bool any = local_experts > 0 && assignments > 0;
@@ -1217,12 +1239,13 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
                          nullptr, 0);
       if (int rc = check_launch("exl3 moe_route")) return rc;
     }
-    auto tile = [&](int projection, int64_t kp, int64_t np, int64_t in_off, int64_t out_off) {
+    // slot: the projection's exponent of each assignment
+    auto tile = [&](int projection, int slot, int64_t kp, int64_t np, int64_t in_off, int64_t out_off) {
       exl3::TileArgs t{};
       t.act = reinterpret_cast<const uint8_t*>(workspace + in_off);
       t.act_row_bytes = 4 * kp;
       t.act_rows = assignments;
-      t.row_exp = reinterpret_cast<const int*>(workspace + lay.ints()) + lay.exps();
+      t.row_exp = reinterpret_cast<const int*>(workspace + lay.ints()) + lay.exps() + slot;
       t.exp_stride = lay.kmax() / 128;
       t.kp = kp;
       t.np = np;
@@ -1259,11 +1282,11 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
     // others one workgroup a row (fewer rows: each row's groups over four
     // wavefronts finish sooner); the register cache sized to the groups a
     // wavefront forms
-    auto form = [&](bool activate, int projection) {
+    auto form = [&](bool activate, int projection, int projections) {
       const int64_t groups = ((activate ? lay.ipad : lay.hpad) / 128 + 3) / 4;
       const int64_t per_wave = (groups + 3) / 4;
-      const dim3 grid{unsigned(assignments), 1u, 1u};
-      const dim3 row_grid{unsigned((assignments + 3) / 4), 1u, 1u};
+      const dim3 grid{unsigned(assignments), unsigned(projections), 1u};
+      const dim3 row_grid{unsigned((assignments + 3) / 4), unsigned(projections), 1u};
 #define VQ_FORM(A, C, W)                                                                            \
   hipLaunchKernelGGL((exl3::moe_form<A, C, W>), W ? row_grid : grid, dim3(256), 0, s, routing, x,   \
                      x_dtype, hidden, intermediate_size, projection, table, workspace, lay,         \
@@ -1288,18 +1311,24 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
 #undef VQ_FORM
       return check_launch("exl3 moe_form");
     };
-    for (int p = 0; p < 2; ++p) {
-      if (int rc = form(false, p)) return rc;
-      const int64_t out_off = p == 0 ? lay.gate() : lay.up();
-      if (int rc = gemv(p, 1, lay.hpad, lay.ipad, lay.input(), 0, out_off, 0)) return rc;
-      if (tiles) {
-        if (int rc = tile(p, lay.hpad, lay.ipad, lay.input(), out_off)) return rc;
+    // gate and up: one form and one GEMV launch for both where the
+    // workspace holds both projections' inputs, else one after the other
+    const int pair =
+        lay.hpad >= exl3::kPairMinHidden && assignments < exl3::kPairMaxSlots && workspace_numel >= lay.total_up() ? 2 : 1;
+    const int64_t in_step = lay.input_up() - lay.input();
+    const int64_t out_step = lay.up() - lay.gate();
+    for (int p = 0; p < 2; p += pair) {
+      if (int rc = form(false, p, pair)) return rc;
+      const int64_t out_off = lay.gate() + p * out_step;
+      if (int rc = gemv(p, pair, lay.hpad, lay.ipad, lay.input(), in_step, out_off, out_step)) return rc;
+      for (int z = 0; tiles && z < pair; ++z) {
+        if (int rc = tile(p + z, z, lay.hpad, lay.ipad, lay.input() + z * in_step, out_off + z * out_step)) return rc;
       }
     }
-    if (int rc = form(true, 2)) return rc;
+    if (int rc = form(true, 2, 1)) return rc;
     if (int rc = gemv(2, 1, lay.ipad, lay.hpad, lay.act(), 0, lay.input(), 0)) return rc;
     if (tiles) {
-      if (int rc = tile(2, lay.ipad, lay.hpad, lay.act(), lay.input())) return rc;
+      if (int rc = tile(2, 0, lay.ipad, lay.hpad, lay.act(), lay.input())) return rc;
     }
   }
   const dim3 combine_grid(unsigned((hidden + exl3::kCombineCols - 1) / exl3::kCombineCols),
