@@ -352,6 +352,34 @@ int marlin_moe_gemm_direct(const void* a_perm, int act_dtype, int64_t a_rows, in
                            void* stream);
 
 /*
+ * The Marlin MoE for calls with many rows per expert, up to the slot rows that
+ * moe_sum adds: the routed slots grouped by expert (no padding) in tasks of at
+ * most task_rows rows, x in the k-permuted layout (marlin_permute_act), then
+ * w13 with the SwiGLU and w2 with the router weight, each expert's weights
+ * dequantized once per task.  The same sums and roundings as
+ * marlin_moe_gemm_direct's kSwiglu and kTopk modes.  No counterpart in the
+ * reference (its prefill path: marlin_moe/prefill.py:381-447).
+ *
+ *   x        [tokens][hidden] of act_dtype, row stride x_stride (a multiple of 8)
+ *   w13, s13 the gate | up matrices and scales of marlin_moe_gemm, N = 2 inter
+ *   w2, s2   the down matrices and scales, K = inter, N = hidden
+ *   topk_ids int32 [tokens * top_k] local experts (outside [0, experts): the
+ *            slot is left out and its c3 row is not written)
+ *   table    int32, marlin_moe_rows_table(tokens * top_k, experts, task_rows)
+ *   xp       [tokens][hidden], h [tokens * top_k][inter], c3 [tokens * top_k]
+ *            [hidden], act_dtype scratch; c3 receives the slot rows
+ * hidden and inter multiples of 128, experts at most 1024, task_rows a
+ * multiple of 16 up to 128; every pointer to x, weights, scales, table and
+ * scratch 16-byte aligned.
+ */
+int64_t marlin_moe_rows_table(int64_t slots, int64_t experts, int64_t task_rows);
+int marlin_moe_rows(const void* x, int act_dtype, int64_t tokens, int64_t x_stride,
+                    const int32_t* w13, const void* s13, const int32_t* w2, const void* s2,
+                    int64_t experts, const int32_t* topk_ids, const float* topk_w, int64_t top_k,
+                    int64_t hidden, int64_t inter, float limit, int64_t task_rows, int32_t* table,
+                    int64_t table_numel, void* xp, void* h, void* c3, void* stream);
+
+/*
  * out[r][p(k)] = a[r][k] for r < rows, k < cols (cols % 32 == 0), p the
  * permutation marlin_moe_gemm_direct reads (inside each 32-k step, k = 8s +
  * 2q + t goes to 8q + 2s + t).  No counterpart in the reference.

@@ -578,3 +578,60 @@ def test_prefill_tile_gemm_matches_oracle_rows(mm, device):
         rw = to_f32(from_f32(np.float32(w.flat[sl]), M.BF16), M.BF16)
         rows[sl] = from_f32(to_f32(y, M.BF16) * rw, M.BF16)
     assert_close(host_bits(c3), rows, M.BF16, "w2 rows")
+
+
+# rows per expert around the 16-row blocks, the 64- and 128-row tasks and the
+# even split above them, none at all, and more than one 2048-slot part
+ROW_COUNTS = [0, 1, 15, 16, 17, 31, 33, 48, 64, 65, 80, 96, 97, 127, 128, 129, 200, 257, 1100]
+
+
+@pytest.mark.parametrize("dtype,limit", [(M.BF16, 7.0), (M.FP16, None)])
+@pytest.mark.parametrize("task_rows", [128, 32])
+@pytest.mark.parametrize("K,N", [(384, 128), (256, 384)])
+def test_rows_path_bitwise_equals_staged(mm, device, dtype, limit, task_rows, K, N):
+    """Grouped row tasks (marlin_moe_rows) against the staged path at one K
+    split: the same MFMA sequence per row and the same roundings, so the
+    slot sums are equal bit for bit; slots of no local expert add nothing."""
+    from vllm_mi355x.kernels.marlin_moe import _C
+    print(f"rows dtype={dtype} task_rows={task_rows} K={K} N={N}", flush=True)
+    rng = np.random.default_rng(K + N + task_rows)
+    E = len(ROW_COUNTS)
+    layer = Layer(rng, E, K, N, dtype, device)
+    flat = rng.permutation(np.concatenate([np.repeat(np.arange(E), ROW_COUNTS), [-1, E, E + 3, -7]]))
+    T, topk = flat.size // 2, 2
+    ids = dev(flat[:2 * T].astype(np.int32).reshape(T, topk), device)
+    w = dev(rng.random((T, topk)).astype(np.float32), device)
+    wide = dev_act(from_f32(rng.standard_normal((T, K + 8)), dtype), dtype, device)
+    x = wide[:, :K]  # rows 8 elements apart
+    want = mm[0].fused_marlin_moe(x, layer.w1, layer.w2, layer.s1, layer.s2, w, ids, clamp_limit=limit,
+                                  block_size=64, ksplit=1, path="staged")
+    slots = T * topk
+    table = torch.full((_C.rows_table(slots, E, task_rows) + 16,), -1, dtype=torch.int32, device=device)
+    act = lambda *shape: torch.full(shape, float("nan"), dtype=x.dtype, device=device)
+    c3 = act(slots, K)
+    _C.rows(x, layer.w1, layer.s1, layer.w2, layer.s2, ids, w.view(-1), topk,
+            math.inf if limit is None else limit, task_rows, table[:-16], act(T, K), act(slots, N), c3)
+    got = mm[1].moe_sum(c3.view(T, topk, K), None, ids, E)
+    torch.cuda.synchronize()
+    assert bool((table[-16:] == -1).all())
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype,limit", [(M.BF16, 10.0), (M.FP16, None)])
+@pytest.mark.parametrize("T", [46, 150])
+def test_many_rows_per_expert_match_oracle(mm, device, dtype, limit, T):
+    """The automatic choice at over 22 rows an expert (row tasks)."""
+    print(f"many rows dtype={dtype} T={T}", flush=True)
+    rng = np.random.default_rng(T + dtype)
+    E, K, N, topk = 4, 256, 128, 2
+    layer = Layer(rng, E, K, N, dtype, device)
+    ids, w = routing(rng, T, E, topk, skew=1.1)
+    ids[3] = [-1, 2]
+    x = from_f32(rng.standard_normal((T, K)), dtype)
+    ws = {}
+    out = mm[0].fused_marlin_moe(dev_act(x, dtype, device), layer.w1, layer.w2, layer.s1, layer.s2,
+                                 dev(w, device), dev(ids, device), clamp_limit=limit, workspace=ws)
+    torch.cuda.synchronize()
+    assert "table" in ws  # the row path ran
+    expected = M.moe(x, dtype, ids, w, *layer.host, limit=math.inf if limit is None else limit)
+    assert_close(host_bits(out), expected, dtype, f"many rows T={T}")

@@ -1781,6 +1781,482 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_permute_kernel(
   *reinterpret_cast<u32x4_t*>(out + r * out_stride + 8 * int64_t(c)) = v;
 }
 
+// ---- many rows per expert: grouped rows, row tiles ------------------------------------
+
+// Calls whose experts hold more rows than an aligned block of the direct path
+// run on row lists of their own (marlin_moe_rows): the routed slots grouped by
+// expert without padding (any order inside an expert: a row's sums depend on
+// nothing but the row), cut into tasks {expert, first row, rows, 0} of at most
+// kRowsTile rows, each expert's tasks of even height in whole 16-row blocks.
+constexpr int kRowsTile = 128;
+constexpr int kRowsPartThreads = 256;
+constexpr int kRowsPartSlots = 8;
+constexpr int kRowsPart = kRowsPartThreads * kRowsPartSlots;  // slots a workgroup counts
+constexpr int kRowsMaxExperts = 1024;
+
+// int32 offsets of the row lists' table: [tasks, 0, 0, 0], the tasks, the
+// sorted slots, then each slot's place in its part (expert << 16 | place, or
+// -1) and the parts' histograms.
+struct RowsLayout {
+  int64_t slots, experts, max_tasks;
+  __host__ __device__ int64_t parts() const { return (slots + kRowsPart - 1) / kRowsPart; }
+  __host__ __device__ int64_t tasks() const { return 4; }
+  __host__ __device__ int64_t sorted() const { return 4 + 4 * max_tasks; }
+  __host__ __device__ int64_t packed() const { return sorted() + (slots + 3) / 4 * 4; }
+  __host__ __device__ int64_t hist() const { return packed() + (slots + 3) / 4 * 4; }
+  __host__ __device__ int64_t total() const { return hist() + parts() * experts; }
+};
+
+// Workgroups 0 .. parts - 1: the experts of kRowsPart slots, each slot's place
+// among the part's rows of its expert, and the part's histogram.  The others:
+// the activations in the k-permuted layout (as moe_align_permute_kernel).
+__global__ __launch_bounds__(kRowsPartThreads) void rows_count_kernel(const int32_t* ids, RowsLayout lay, int32_t* table,
+                                                                      const uint16_t* a, int64_t a_stride,
+                                                                      int64_t rows, int cols, uint16_t* out) {
+  extern __shared__ int part_count[];
+  const int experts = int(lay.experts);
+  const int64_t parts = lay.parts();
+  if (blockIdx.x >= parts) {
+    const int64_t i = int64_t(blockIdx.x - parts) * kRowsPartThreads + threadIdx.x;
+    const int64_t per_row = int64_t(cols) / 8;
+    if (i >= rows * per_row) return;
+    const int64_t r = i / per_row;
+    const int c = int(i - r * per_row);
+    const uint16_t* src = a + r * a_stride + (c >> 2) * 32 + 2 * (c & 3);
+    u32x4_t v;
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) v[s4] = *reinterpret_cast<const uint32_t*>(src + 8 * s4);
+    *reinterpret_cast<u32x4_t*>(out + r * cols + 8 * int64_t(c)) = v;
+    return;
+  }
+  for (int e = threadIdx.x; e < experts; e += kRowsPartThreads) part_count[e] = 0;
+  __syncthreads();
+  const int64_t s0 = int64_t(blockIdx.x) * kRowsPart + threadIdx.x;
+  int e[kRowsPartSlots];
+#pragma unroll
+  for (int u = 0; u < kRowsPartSlots; ++u) {
+    const int64_t slot = s0 + u * kRowsPartThreads;
+    const int id = slot < lay.slots ? ids[slot] : -1;
+    e[u] = id >= 0 && id < experts ? id : -1;
+  }
+#pragma unroll
+  for (int u = 0; u < kRowsPartSlots; ++u) {
+    const int64_t slot = s0 + u * kRowsPartThreads;
+    const int v = e[u] >= 0 ? (e[u] << 16) | atomicAdd(&part_count[e[u]], 1) : -1;
+    if (slot < lay.slots) table[lay.packed() + slot] = v;
+  }
+  __syncthreads();
+  for (int x = threadIdx.x; x < experts; x += kRowsPartThreads) {
+    table[lay.hist() + int64_t(blockIdx.x) * experts + x] = part_count[x];
+  }
+}
+
+// Tasks of an expert of c rows, and the rows of each but the last.
+__device__ __forceinline__ int rows_tasks(int c, int task_rows) { return (c + task_rows - 1) / task_rows; }
+__device__ __forceinline__ int rows_height(int c, int tasks) {
+  return tasks > 0 ? ((c + tasks - 1) / tasks + 15) / 16 * 16 : 16;
+}
+
+// One workgroup per part: every expert's first row (a scan of the summed
+// histograms, the same in each workgroup) plus the rows of the parts before
+// this one place the part's slots; workgroup 0 also writes the tasks.  Experts
+// e0 .. e1 - 1 (a contiguous run) belong to one thread.
+__global__ __launch_bounds__(kRowsPartThreads) void rows_fill_kernel(RowsLayout lay, int32_t* table, int task_rows) {
+  extern __shared__ int first[];  // experts: where this part's rows of the expert begin
+  __shared__ int wave_rows[kRowsPartThreads / 64], wave_tasks[kRowsPartThreads / 64];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int experts = int(lay.experts);
+  const int parts = int(lay.parts());
+  const int part = int(blockIdx.x);
+  const int per = (experts + kRowsPartThreads - 1) / kRowsPartThreads;
+  constexpr int kPer = kRowsMaxExperts / kRowsPartThreads;
+  const int e0 = tid * per;
+  int total[kPer], before[kPer];
+  int rows = 0, tasks = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    total[i] = before[i] = 0;
+    const int e = e0 + i;
+    if (i < per && e < experts) {
+      for (int p0 = 0; p0 < parts; p0 += 8) {
+        int n[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          n[u] = p0 + u < parts ? table[lay.hist() + int64_t(p0 + u) * experts + e] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          total[i] += n[u];
+          if (p0 + u < part) before[i] += n[u];
+        }
+      }
+      rows += total[i];
+      const int h = rows_height(total[i], rows_tasks(total[i], task_rows));
+      tasks += rows_tasks(total[i], h);
+    }
+  }
+  int irows = rows, itasks = tasks;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int r = __shfl_up(irows, d), t = __shfl_up(itasks, d);
+    if (lane >= d) {
+      irows += r;
+      itasks += t;
+    }
+  }
+  if (lane == 63) {
+    wave_rows[wave] = irows;
+    wave_tasks[wave] = itasks;
+  }
+  __syncthreads();
+  int row = irows - rows, task = itasks - tasks;
+  for (int w = 0; w < wave; ++w) {
+    row += wave_rows[w];
+    task += wave_tasks[w];
+  }
+  if (part == 0 && tid == kRowsPartThreads - 1) table[0] = task + tasks;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int e = e0 + i;
+    if (i < per && e < experts) {
+      first[e] = row + before[i];
+      if (part == 0) {
+        const int h = rows_height(total[i], rows_tasks(total[i], task_rows));
+        for (int r = 0; r < total[i]; r += h) {
+          reinterpret_cast<int4*>(table + lay.tasks())[task++] = make_int4(e, row + r, min(h, total[i] - r), 0);
+        }
+      }
+      row += total[i];
+    }
+  }
+  __syncthreads();
+  const int64_t s0 = int64_t(part) * kRowsPart + tid;
+  int v[kRowsPartSlots];
+#pragma unroll
+  for (int u = 0; u < kRowsPartSlots; ++u) {
+    const int64_t slot = s0 + u * kRowsPartThreads;
+    v[u] = slot < lay.slots ? table[lay.packed() + slot] : -1;
+  }
+#pragma unroll
+  for (int u = 0; u < kRowsPartSlots; ++u) {
+    if (v[u] >= 0) table[lay.sorted() + first[v[u] >> 16] + (v[u] & 0xffff)] = int(s0 + u * kRowsPartThreads);
+  }
+}
+
+struct RowsArgs {
+  const uint16_t* a;      // k-permuted rows of K: tokens (w13), sorted rows (w2)
+  uint32_t a_bytes;
+  const u32x4_t* w;       // [E][K/16][N/2] 16-byte fragments
+  const uint16_t* s;      // [E][K/128][N] group scales
+  const int32_t* table;
+  int64_t tasks, sorted;  // offsets in the table
+  const float* topk_w;    // w2: [slots]
+  uint16_t* out;          // w13: h [sorted row][N / 2], k-permuted; w2: [slot][N]
+  int top_k, K, N;
+  int cols;               // column groups (workgroups) per task
+  float limit;
+};
+
+typedef __attribute__((address_space(3))) void* rows_lds_t;
+
+// LDS reads the compiler does not see (it would make each wait for every
+// LDS-DMA load in flight); a value is ready after rows_lgkm and rows_ready.
+template <int kOffset>
+__device__ __forceinline__ void rows_read(u32x4_t& v, uint32_t address) {
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(address), "i"(kOffset));
+}
+template <int n>
+__device__ __forceinline__ void rows_lgkm() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(n));
+}
+__device__ __forceinline__ void rows_ready(u32x4_t& v) { asm volatile("" : "+v"(v)); }
+
+// f(std::integral_constant<int, i>) for i = 0 .. n - 1.
+template <int n, int i = 0, typename F>
+__device__ __forceinline__ void rows_for(F&& f) {
+  if constexpr (i < n) {
+    f(std::integral_constant<int, i>{});
+    rows_for<n, i + 1>(f);
+  }
+}
+
+// One workgroup = (task of up to 128 rows, 256 columns), a wavefront 64 columns
+// (kSwiglu: wavefronts 0, 1 gate tiles and 2, 3 the up tiles N / 128 further
+// on).  Per 32-k step a wavefront dequantizes its 2048 weights once for all the
+// task's rows, one step ahead of their MFMAs (A operands as marlin_gemm's, the
+// same MFMA sequence per row, so the sums are bitwise its at one K split); the
+// rows' operands and the weights come by LDS-DMA, rows 2 steps and weights 4
+// steps ahead, one barrier a step.
+// What bounds it: the matrix pipe and the dequant share the SIMD's issue (512
+// cycles of MFMA and about 300 of BF16 dequant a step at 128 rows), so the rows
+// per dequant set the rate.
+// Workgroups go to the 8 XCDs round robin: XCD x runs tasks x, x + 8, ..., all
+// column groups of a task one after another, so its L2 fetches the task's rows
+// once.
+template <bool kBF16, bool kSwiglu>
+__global__ __launch_bounds__(kThreads, 2) void marlin_gemm_rows(RowsArgs g) {
+  constexpr int kSubs = kRowsTile / 16;
+  constexpr int kABuf = kSubs * 1024;   // one step of the rows: [16-row block][q][row] 16 bytes
+  constexpr int kABufs = 3;
+  constexpr int kRing = 4;              // weight steps, 1 KB per wavefront each
+  constexpr int kABytes = kABufs * kABuf;
+  constexpr int kWBytes = 4 * kRing * 1024;
+  constexpr int kSBytes = 4 * 2 * 256;  // two group-scale slots per wavefront (128 bytes used)
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kABytes + kWBytes + kSBytes];
+  static_assert(4 * 2 * 4096 <= kABytes + kWBytes, "two sub-blocks of every wavefront's sums fit for the exchange");
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = vq::uniform(tid >> 6);
+  const int q = lane >> 4;
+  const int col = lane & 15;
+  const int local = int(blockIdx.x >> 3);
+  const int task = local / g.cols * 8 + int(blockIdx.x & 7);
+  const int cgrp = local % g.cols;
+  if (task >= g.table[0]) return;
+  const int4 tk = reinterpret_cast<const int4*>(g.table + g.tasks)[task];
+  const int e = vq::uniform(tk.x);
+  const int first = vq::uniform(tk.y);
+  const int nrows = vq::uniform(tk.z);
+  const int32_t* sorted = g.table + g.sorted + first;
+  int tile;
+  bool tile_ok;
+  if constexpr (kSwiglu) {
+    const int gate_tiles = g.N >> 7;
+    const int gt = 2 * cgrp + (wave & 1);
+    tile = wave < 2 ? gt : gate_tiles + gt;
+    tile_ok = gt < gate_tiles;
+  } else {
+    tile = 4 * cgrp + wave;
+    tile_ok = tile < (g.N >> 6);
+  }
+  if (!tile_ok) tile = 0;  // a missing tile streams tile 0 and stores nothing
+
+  const int steps = g.K >> 5;
+  const int last = steps - 1;
+  const uint32_t wstep = uint32_t(g.N) * 16u;
+  const __amdgpu_buffer_rsrc_t wbuf =
+      buffer(g.w + int64_t(e) * (g.K >> 4) * (g.N >> 1), uint32_t(g.K >> 4) * uint32_t(g.N >> 1) * 16u);
+  const __amdgpu_buffer_rsrc_t sbuf =
+      buffer(g.s + int64_t(e) * (g.K >> 7) * g.N, uint32_t(g.K >> 7) * uint32_t(g.N) * 2u);
+  const __amdgpu_buffer_rsrc_t abuf = buffer(g.a, g.a_bytes);
+  const int woff = int(fragment_offset(g.N, tile, lane));
+  // the tile's 64 group scales: a dword in each of lanes 0-31 (the others read
+  // past the buffer: zeros, into the slot's unread half)
+  const int soff = lane < 32 ? int(tile * 128 + 4 * lane) : int(0x80000000u);
+  // rows: this wavefront copies 16-row blocks 2 wave, 2 wave + 1 (rows past the
+  // task repeat its last row)
+  int aoff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int t = min(16 * (2 * wave + i) + col, nrows - 1);
+    const int row = kSwiglu ? sorted[t] / g.top_k : first + t;
+    aoff[i] = int(uint32_t(row) * uint32_t(g.K) * 2u) + 16 * q;
+  }
+  auto load_rows = [&](int s) {
+    const int from = min(s, last);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int voff = aoff[i];
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(abuf, (rows_lds_t)&lds[s % kABufs * kABuf + (2 * wave + i) * 1024], 16,
+                                               voff, from * 64, 0, 0);
+    }
+  };
+  auto load_weights = [&](int s) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, (rows_lds_t)&lds[kABytes + (wave * kRing + s % kRing) * 1024], 16,
+                                             woff, int(uint32_t(min(s, last)) * wstep), 0, 0);
+  };
+  auto load_scales = [&](int group) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(sbuf, (rows_lds_t)&lds[kABytes + kWBytes + (wave * 2 + (group & 1)) * 256], 4,
+                                             soff, int(uint32_t(min(group, last >> 2)) * uint32_t(g.N) * 2u), 0, 0);
+  };
+  const uint32_t a_lane = vq::lds_address(&lds[0]) + 16 * lane;
+  const uint32_t w_lane = vq::lds_address(&lds[kABytes]) + wave * kRing * 1024 + 16 * lane;
+  const uint32_t s_lane = vq::lds_address(&lds[kABytes + kWBytes]) + wave * 512 + 16 * (lane & 7);
+  NibbleMasks masks;
+  masks.lo = 0x000f000fu;
+  masks.hi = 0x00f000f0u;
+  masks.magic = 0x64006400u;
+  Scales<kBF16> sc;
+
+  auto run = [&](auto ns_tag) __attribute__((always_inline)) {
+    constexpr int kNs = decltype(ns_tag)::value;
+    f32x4_t acc[4][kNs];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int sb = 0; sb < kNs; ++sb) acc[j][sb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    u32x4_t wcur[4];
+    // Order of the loads: step s issues [S(s / 4 + 1) where s % 4 == 0] A(s + 2)
+    // W(s + 4), A two loads; before step 0 the same order from step -4 on.
+    asm volatile("" ::: "memory");
+    load_scales(0);
+    load_weights(0);
+    load_weights(1);
+    load_rows(0);
+    load_weights(2);
+    load_rows(1);
+    load_weights(3);
+    vq::wait_vmcnt<4>();  // S(0), W(0), W(1) and A(0) landed (after them: W(2), A(1), W(3))
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    {
+      u32x4_t wv, sv;
+      rows_read<0>(wv, w_lane);
+      rows_read<0>(sv, s_lane);
+      rows_lgkm<0>();
+      rows_ready(wv);
+      rows_ready(sv);
+      sc.set(sv, lane);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t word = wv[j];
+        wcur[j] = sc.operand(combine(word, lane), j, masks);
+      }
+    }
+    auto step = [&](int s, auto slot) __attribute__((always_inline)) {
+      constexpr int kS = decltype(slot)::value;  // s % 4
+      if constexpr (kS == 0) load_scales((s >> 2) + 1);
+      load_rows(s + 2);
+      // W(s + 1) landed: after it came A(s), W(s + 2), A(s + 1), W(s + 3), A(s + 2)
+      // (and at most one S, not counted: a stricter wait)
+      vq::wait_vmcnt<8>();
+      u32x4_t wv, sv;
+      rows_read<(kS + 1) % kRing * 1024>(wv, w_lane);  // (past the last step: unused)
+      if constexpr (kS == 3) rows_read<0>(sv, s_lane + uint32_t(((s >> 2) + 1) & 1) * 256);
+      load_weights(s + 4);
+      const uint32_t a_buf = a_lane + uint32_t(s % kABufs) * kABuf;
+      u32x4_t b[kNs];
+      rows_read<0>(b[0], a_buf);
+      if constexpr (kNs > 1) rows_read<1024>(b[1], a_buf);
+      u32x4_t wnext[4];
+      rows_for<kNs>([&](auto sb_tag) __attribute__((always_inline)) {
+        constexpr int sb = decltype(sb_tag)::value;
+        rows_lgkm<(sb + 1 < kNs ? 1 : 0)>();  // the read of sub-block sb + 1 may be pending
+        rows_ready(b[sb]);
+        if constexpr (sb == 0) {
+          rows_ready(wv);
+          if constexpr (kS == 3) rows_ready(sv);
+        }
+        if constexpr (sb + 2 < kNs) rows_read<(sb + 2) * 1024>(b[sb + 2], a_buf);
+        if constexpr (sb == 0) {
+          if constexpr (kS == 3) sc.set(sv, lane);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t word = wv[j];
+            wnext[j] = sc.operand(combine(word, lane), j, masks);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j][sb] = mfma<kBF16>(wcur[j], b[sb], acc[j][sb]);
+      });
+#pragma unroll
+      for (int j = 0; j < 4; ++j) wcur[j] = wnext[j];
+      // A(s + 1) of this wavefront landed: after it came W(s + 3), A(s + 2), W(s + 4)
+      // (an S not counted); then every wavefront's, and every read of buffer s done
+      vq::wait_vmcnt<4>();
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    for (int s = 0; s < steps; s += 4) {
+      step(s, std::integral_constant<int, 0>{});
+      step(s + 1, std::integral_constant<int, 1>{});
+      step(s + 2, std::integral_constant<int, 2>{});
+      step(s + 3, std::integral_constant<int, 3>{});
+    }
+    // the clamped loads past the last step may still be landing
+    vq::wait_vmcnt<0>();
+    __syncthreads();
+
+    if constexpr (kSwiglu) {
+      // gate wavefront w and up wavefront w + 2 share the h of their tile: of
+      // every four 16-row blocks the gate wavefront finishes the first two and
+      // the up wavefront the last two, each handing the other's sums over
+      // through LDS
+      auto xch = [&](int w, int j, int i) {
+        return reinterpret_cast<f32x4_t*>(lds) + ((w * 2 + i) * 4 + j) * 64 + lane;
+      };
+      const bool gate = wave < 2;
+      const int tile_h = 2 * cgrp + (wave & 1);
+#pragma unroll
+      for (int r0 = 0; r0 < kNs; r0 += 4) {
+        if (r0 > 0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if (gate) {
+              if (r0 + 2 + i < kNs) *xch(wave, j, i) = acc[j][r0 + 2 + i < kNs ? r0 + 2 + i : 0];
+            } else {
+              if (r0 + i < kNs) *xch(wave, j, i) = acc[j][r0 + i < kNs ? r0 + i : 0];
+            }
+          }
+        __syncthreads();
+        if (!tile_ok) continue;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int sbg = r0 + i < kNs ? r0 + i : 0, sbu = r0 + 2 + i < kNs ? r0 + 2 + i : 0;
+          const bool on = gate ? r0 + i < kNs : r0 + 2 + i < kNs;
+          const int t = 16 * (gate ? r0 + i : r0 + 2 + i) + col;
+          if (!on || t >= nrows) continue;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const f32x4_t own = gate ? acc[j][sbg] : acc[j][sbu];
+            const f32x4_t other = *xch(wave ^ 2, j, i);
+            uint16_t hv[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const float o = own[c], p = other[c];
+              hv[c] = swiglu<kBF16>(gate ? o : p, gate ? p : o, g.limit);
+            }
+            // columns n .. n + 3: two adjacent pairs in the permuted layout
+            const int n = tile_h * 64 + 16 * j + 4 * q;
+            uint16_t* row = g.out + int64_t(first + t) * (g.N >> 1);
+            *reinterpret_cast<uint32_t*>(row + permuted_k(n)) = uint32_t(hv[0]) | (uint32_t(hv[1]) << 16);
+            *reinterpret_cast<uint32_t*>(row + permuted_k(n + 2)) = uint32_t(hv[2]) | (uint32_t(hv[3]) << 16);
+          }
+        }
+      }
+    } else {
+      if (!tile_ok) return;
+      // the slots and their router weights before the first store (loads and
+      // stores share one in-order counter)
+      int slots[kNs];
+      float wts[kNs];
+#pragma unroll
+      for (int sb = 0; sb < kNs; ++sb) {
+        const int t = 16 * sb + col;
+        slots[sb] = t < nrows ? sorted[t] : -1;
+        wts[sb] = t < nrows ? round_act<kBF16>(g.topk_w[slots[sb]]) : 0.0f;
+      }
+#pragma unroll
+      for (int sb = 0; sb < kNs; ++sb) {
+        if (slots[sb] < 0) continue;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4_t v = acc[j][sb];
+          float x[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) x[u] = round_act<kBF16>(v[u]) * wts[sb];  // exact product
+          const u32x2_t packed = {uint32_t(to_act<kBF16>(x[0])) | (uint32_t(to_act<kBF16>(x[1])) << 16),
+                                  uint32_t(to_act<kBF16>(x[2])) | (uint32_t(to_act<kBF16>(x[3])) << 16)};
+          *reinterpret_cast<u32x2_t*>(g.out + int64_t(slots[sb]) * g.N + tile * 64 + 16 * j + 4 * q) = packed;
+        }
+      }
+    }
+  };
+  const int nsub = (nrows + 15) >> 4;
+  if (nsub <= 1) run(std::integral_constant<int, 1>{});
+  else if (nsub == 2) run(std::integral_constant<int, 2>{});
+  else if (nsub == 3) run(std::integral_constant<int, 3>{});
+  else if (nsub == 4) run(std::integral_constant<int, 4>{});
+  else if (nsub == 5) run(std::integral_constant<int, 5>{});
+  else if (nsub == 6) run(std::integral_constant<int, 6>{});
+  else run(std::integral_constant<int, 8>{});
+}
+
 // ---- host ----------------------------------------------------------------------------
 
 template <bool kBF16, int kTilesWG, int kSub>
@@ -2084,6 +2560,97 @@ extern "C" int marlin_moe_gemm_direct(const void* a_perm, int act_dtype, int64_t
   const hipStream_t s = static_cast<hipStream_t>(stream);
   return act_dtype == vq::kBF16 ? marlin::dispatch_direct<true>(g, mode, int(blocks), int(ksplit), s)
                                 : marlin::dispatch_direct<false>(g, mode, int(blocks), int(ksplit), s);
+}
+
+extern "C" int64_t marlin_moe_rows_table(int64_t slots, int64_t experts, int64_t task_rows) {
+  if (slots < 0 || slots > INT_MAX || experts <= 0 || experts > marlin::kRowsMaxExperts || task_rows < 16 ||
+      task_rows > marlin::kRowsTile || task_rows % 16 != 0) {
+    vq::fail("marlin rows: slots, experts (at most 1024) or task rows (16 .. 128, whole 16s) out of range");
+    return -1;
+  }
+  return marlin::RowsLayout{slots, experts, slots / 16 + std::min(experts, slots)}.total();
+}
+
+extern "C" int marlin_moe_rows(const void* x, int act_dtype, int64_t tokens, int64_t x_stride, const int32_t* w13,
+                               const void* s13, const int32_t* w2, const void* s2, int64_t experts,
+                               const int32_t* topk_ids, const float* topk_w, int64_t top_k, int64_t hidden,
+                               int64_t inter, float limit, int64_t task_rows, int32_t* table, int64_t table_numel,
+                               void* xp, void* h, void* c3, void* stream) {
+  using namespace vq;
+  using namespace marlin;
+  if (act_dtype != kBF16 && act_dtype != kFP16) return fail("a: bf16 or fp16 activations");
+  if (hidden <= 0 || inter <= 0 || hidden % 128 != 0 || inter % 128 != 0) return fail("marlin rows: hidden % 128, inter % 128");
+  if (tokens < 0 || top_k <= 0 || tokens > INT_MAX / top_k) return fail("routing sizes out of range");
+  const int64_t slots = tokens * top_k;
+  const int64_t need = marlin_moe_rows_table(slots, experts, task_rows);
+  if (need < 0) return kInvalidArgument;
+  if (table_numel < need) return fail("marlin rows: table too small");
+  if (x_stride < hidden || x_stride % 8 != 0) return fail("a: unit inner stride, row stride a multiple of 8 and at least K");
+  if (tokens * hidden * 2 >= (int64_t(1) << 31) || slots * inter * 2 >= (int64_t(1) << 31) ||
+      hidden * inter >= (int64_t(1) << 31)) {
+    return fail("a and each expert's weights must stay below 2 GiB");
+  }
+  if (!aligned16(x) || !aligned16(w13) || !aligned16(s13) || !aligned16(w2) || !aligned16(s2) || !aligned16(table) ||
+      !aligned16(xp) || !aligned16(h) || !aligned16(c3)) {
+    return fail("a, w and s must be 16-byte aligned");
+  }
+  if (!topk_ids || !topk_w) return fail("topk weights required");
+  if (std::isnan(limit)) return fail("act: limit must not be NaN");
+  if (slots == 0) return kOk;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const RowsLayout lay{slots, experts, slots / 16 + std::min(experts, slots)};
+  const int64_t chunks = tokens * (hidden / 8);
+  const int64_t groups = lay.parts() + (chunks + kRowsPartThreads - 1) / kRowsPartThreads;
+  // an expert of c rows has at most ceil(c / task_rows) tasks
+  const int64_t bound = slots / task_rows + std::min(experts, slots);
+  const int64_t cols13 = (inter / 64 + 1) / 2;
+  const int64_t cols2 = (hidden / 64 + 3) / 4;
+  const int64_t per_xcd = (bound + 7) / 8;
+  if (groups > INT_MAX || 8 * per_xcd * std::max(cols13, cols2) > INT_MAX) return fail("marlin rows: too many rows");
+  hipLaunchKernelGGL(rows_count_kernel, dim3(unsigned(groups)), dim3(kRowsPartThreads), size_t(experts) * sizeof(int), st,
+                     topk_ids, lay, table, static_cast<const uint16_t*>(x), x_stride, tokens, int(hidden),
+                     static_cast<uint16_t*>(xp));
+  if (int rc = check_launch("marlin rows_count")) return rc;
+  hipLaunchKernelGGL(rows_fill_kernel, dim3(unsigned(lay.parts())), dim3(kRowsPartThreads), size_t(experts) * sizeof(int), st,
+                     lay, table, int(task_rows));
+  if (int rc = check_launch("marlin rows_fill")) return rc;
+  RowsArgs a{};
+  a.a = static_cast<const uint16_t*>(xp);
+  a.a_bytes = uint32_t(tokens * hidden * 2);
+  a.w = reinterpret_cast<const u32x4_t*>(w13);
+  a.s = static_cast<const uint16_t*>(s13);
+  a.table = table;
+  a.tasks = lay.tasks();
+  a.sorted = lay.sorted();
+  a.topk_w = topk_w;
+  a.out = static_cast<uint16_t*>(h);
+  a.top_k = int(top_k);
+  a.K = int(hidden);
+  a.N = int(2 * inter);
+  a.cols = int(cols13);
+  a.limit = limit;
+  const dim3 grid13(unsigned(8 * per_xcd * cols13));
+  if (act_dtype == kBF16) {
+    hipLaunchKernelGGL((marlin_gemm_rows<true, true>), grid13, dim3(kThreads), 0, st, a);
+  } else {
+    hipLaunchKernelGGL((marlin_gemm_rows<false, true>), grid13, dim3(kThreads), 0, st, a);
+  }
+  if (int rc = check_launch("marlin_gemm_rows w13")) return rc;
+  a.a = static_cast<const uint16_t*>(h);
+  a.a_bytes = uint32_t(slots * inter * 2);
+  a.w = reinterpret_cast<const u32x4_t*>(w2);
+  a.s = static_cast<const uint16_t*>(s2);
+  a.out = static_cast<uint16_t*>(c3);
+  a.K = int(inter);
+  a.N = int(hidden);
+  a.cols = int(cols2);
+  const dim3 grid2(unsigned(8 * per_xcd * cols2));
+  if (act_dtype == kBF16) {
+    hipLaunchKernelGGL((marlin_gemm_rows<true, false>), grid2, dim3(kThreads), 0, st, a);
+  } else {
+    hipLaunchKernelGGL((marlin_gemm_rows<false, false>), grid2, dim3(kThreads), 0, st, a);
+  }
+  return check_launch("marlin_gemm_rows w2");
 }
 
 extern "C" int marlin_permute_act(const void* a, int act_dtype, int64_t rows, int64_t cols, int64_t a_stride,

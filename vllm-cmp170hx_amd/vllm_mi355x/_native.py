@@ -92,6 +92,15 @@ SIGNATURES = {
         c_vp, c_i64, c_vp, c_i64, c_i64,      # part, part_numel, out, out_stride, out_rows
         c_vp,                                 # stream
     ]),
+    "marlin_moe_rows_table": (c_i64, [c_i64, c_i64, c_i64]),
+    "marlin_moe_rows": (c_int, [
+        c_vp, c_int, c_i64, c_i64,            # x, act_dtype, tokens, x_stride
+        c_vp, c_vp, c_vp, c_vp, c_i64,        # w13, s13, w2, s2, experts
+        c_vp, c_vp, c_i64,                    # topk_ids, topk_w, top_k
+        c_i64, c_i64, ctypes.c_float, c_i64,  # hidden, inter, limit, task_rows
+        c_vp, c_i64,                          # table, table_numel
+        c_vp, c_vp, c_vp, c_vp,               # xp, h, c3, stream
+    ]),
     "marlin_permute_act": (c_int, [c_vp, c_int, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp]),
     "marlin_moe_align_permute": (c_int, [
         c_vp, c_i64, c_i64, c_i64, c_vp,      # topk_ids, numel, num_experts, block_size, expert_map

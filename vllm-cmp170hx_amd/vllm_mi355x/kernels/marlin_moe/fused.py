@@ -63,6 +63,18 @@ def workspace_shapes(tokens: int, topk: int, hidden: int, inter: int, experts: i
     return shapes
 
 
+# Tokens per aligned block the direct path takes at most; calls whose experts
+# hold more rows than that (over 22 on average, choose_block_size) run on row
+# lists (marlin_moe_rows), whose tasks hold up to 128 rows per dequantized weight.
+# Both sides measured, us per call in BF16 / FP16, 128 experts of 2048 / 768 at
+# top-8: 16 rows an expert, direct 130 / 93, rows 141 / 114; 25 rows, staged blocks
+# of 64 (what such calls ran on) 166 / 140, rows 142 / 118; 128 rows 442 / 376 and
+# 292 / 262.  Tasks of 128 rows were the best or within 5% of it from 25 to 512
+# rows an expert (64: 340 / 285 at 128 rows) but for 16 experts of 128 rows (96: 173
+# against 202).
+_DIRECT_MAX_BLOCK = 32
+_TASK_ROWS = 128
+
 # workgroups the direct w13 must have to be chosen (tuned on MI355X)
 _DIRECT_MIN_WORKGROUPS = 384
 
@@ -79,6 +91,26 @@ def direct_applies(tokens: int, topk: int, hidden: int, inter: int, experts: int
     slots = tokens * topk
     touched = experts * (1.0 - (1.0 - 1.0 / max(experts, 1)) ** slots)
     return touched * (2 * inter // 256) >= _DIRECT_MIN_WORKGROUPS
+
+
+def rows_task_rows(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
+                   w1_scale: torch.Tensor, w2_scale: torch.Tensor, topk: int) -> int:
+    """Rows per task of the many-rows path (marlin_moe_rows) for a call, or 0
+    where it does not apply (the staged path's own checks then answer): whole
+    128-column gate / up pairs, at most 1024 experts, 16-byte aligned contiguous
+    weights and rows, 32-bit offsets."""
+    M, K = hidden_states.shape
+    E, N = w1.size(0), w2.size(1) * 16
+    slots = M * topk
+    if (K % 128 != 0 or N % 128 != 0 or E > 1024 or hidden_states.stride(1) != 1
+            or hidden_states.stride(0) % 8 != 0 or M * hidden_states.stride(0) >= 1 << 30
+            or slots * max(K, N) >= 1 << 30 or K * N >= 1 << 31):
+        return 0
+    tensors = (hidden_states, w1, w2, w1_scale, w2_scale)
+    if any(t.data_ptr() % 16 for t in tensors) or any(
+            not t.is_contiguous() or t.device != hidden_states.device for t in tensors[1:]):
+        return 0
+    return _TASK_ROWS
 
 
 def marlin_dequant(w: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
@@ -112,7 +144,9 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
     1) or "split" (the staged kernels over the split-cover block lists of
     split_align: one w13 and one w2 launch per list, as the reference's
     prefill.run, marlin_moe/prefill.py:381-447).  All give the same sums: a
-    row's sums depend only on its own activations, expert and K split."""
+    row's sums depend only on its own activations, expert and K split.  The
+    automatic choice also takes row lists for calls with many rows per expert
+    (_rows_path; K split 1)."""
     M, K = hidden_states.shape
     E = w1.size(0)
     N = w2.size(1) * 16
@@ -138,6 +172,11 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
         inside = (ids >= 0) & (ids < emap.numel())
         local = torch.where(inside, emap[torch.where(inside, ids, 0).long()], -1).contiguous()
     bs = block_size or choose_block_size(M, topk, E)
+    if path is None and block_size is None and ksplit is None and bs > _DIRECT_MAX_BLOCK:
+        task_rows = rows_task_rows(hidden_states, w1, w2, w1_scale, w2_scale, topk)
+        if task_rows:
+            return _rows_path(hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, local, out,
+                              limit, task_rows, workspace)
     if path is None:
         direct = ksplit in (None, 1) and direct_applies(M, topk, K, N, E, bs)
     elif path == "split":
@@ -197,6 +236,33 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
         return out
     _C.gemm(buf["h"], w2, w2_scale, sorted_ids, expert_ids, ntpp, tw, 1, slots,
             N, K, bs, _C.MODE_TOPK, 1, out=buf["c3"])
+    moe_sum(buf["c3"].view(M, topk, K), out, local, E)
+    return out
+
+
+def _rows_path(hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, local, out, limit,
+               task_rows, workspace):
+    """Many rows per expert: the slots grouped by expert in tasks of task_rows
+    rows, each task's weights dequantized once (marlin_moe_rows)."""
+    M, K = hidden_states.shape
+    N, E = w2.size(1) * 16, w1.size(0)
+    topk = local.size(1)
+    slots = M * topk
+    ws = workspace if workspace is not None else {}
+    buf = {}
+    for name, shape, dtype in (("table", (_C.rows_table(slots, E, task_rows),), torch.int32),
+                               ("xp", (M, K), hidden_states.dtype),
+                               ("h", (slots, N), hidden_states.dtype),
+                               ("c3", (slots, K), hidden_states.dtype)):
+        t = ws.get(name)
+        numel = math.prod(shape)
+        if t is None or t.numel() < numel or t.dtype != dtype:
+            t = torch.empty(numel, dtype=dtype, device=hidden_states.device)
+            ws[name] = t
+        buf[name] = t.view(-1)[:numel].view(shape)
+    tw = topk_weights.to(torch.float32).contiguous().view(-1)
+    _C.rows(hidden_states, w1, w1_scale, w2, w2_scale, local, tw, topk, limit, task_rows,
+            buf["table"], buf["xp"], buf["h"], buf["c3"])
     moe_sum(buf["c3"].view(M, topk, K), out, local, E)
     return out
 
