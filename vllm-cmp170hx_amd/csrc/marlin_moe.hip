@@ -133,8 +133,12 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 // BF16: (q - 8) * s is exact in FP32 (4 x 8 significant bits), so
 // fma(q, s, -8 s) is that product and the conversion rounds once.
 __device__ __forceinline__ void dequant_bf16(uint32_t c, float s, float ns8, uint32_t (&o)[4]) {
-  const uint32_t lo = c & 0x0f0f0f0fu;         // [2q, 16+2q, 2q+1, 17+2q]
-  const uint32_t hi = (c >> 4) & 0x0f0f0f0fu;  // [2q+8, 24+2q, 2q+9, 25+2q]
+  uint32_t lo = c & 0x0f0f0f0fu;         // [2q, 16+2q, 2q+1, 17+2q]
+  uint32_t hi = (c >> 4) & 0x0f0f0f0fu;  // [2q+8, 24+2q, 2q+9, 25+2q]
+  // (the values hidden from the compiler: knowing each byte's high nibble zero,
+  // it would extract three of every four bytes with a v_bfe_u32 before the
+  // conversion, instead of converting byte 1, 2 or 3 in place)
+  asm("" : "+v"(lo), "+v"(hi));
   auto two = [&](uint32_t w, int b0, int b1) {
     const float x0 = __builtin_fmaf(float((w >> (8 * b0)) & 0xffu), s, ns8);
     const float x1 = __builtin_fmaf(float((w >> (8 * b1)) & 0xffu), s, ns8);
@@ -156,7 +160,7 @@ __device__ __forceinline__ uint32_t fragment_offset(int N, int tile, int lane) {
 
 // Swap with lane r ^ 8 of the 16-lane row and keep this lane's column's bytes.
 __device__ __forceinline__ uint32_t combine(uint32_t own, int lane) {
-  const uint32_t other = uint32_t(__builtin_amdgcn_update_dpp(0, int(own), 0x128, 0xf, 0xf, false));
+  const uint32_t other = uint32_t(__builtin_amdgcn_mov_dpp(int(own), 0x128, 0xf, 0xf, true));
   // r < 8: own = row A, half 0 (bytes 0, 2); r >= 8: own = row B, half 1 (bytes 1, 3)
   return __builtin_amdgcn_perm(other, own, (lane & 8) ? 0x03070105u : 0x06020400u);
 }
