@@ -608,10 +608,10 @@ def test_rows_path_bitwise_equals_staged(mm, device, dtype, limit, task_rows, K,
     slots = T * topk
     table = torch.full((_C.rows_table(slots, E, task_rows) + 16,), -1, dtype=torch.int32, device=device)
     act = lambda *shape: torch.full(shape, float("nan"), dtype=x.dtype, device=device)
-    c3 = act(slots, K)
-    _C.rows(x, layer.w1, layer.s1, layer.w2, layer.s2, ids, w.view(-1), topk,
-            math.inf if limit is None else limit, task_rows, table[:-16], act(T, K), act(slots, N), c3)
-    got = mm[1].moe_sum(c3.view(T, topk, K), None, ids, E)
+    got = act(T, K)
+    _C.fused(x, layer.w1, layer.w2, layer.s1, layer.s2, w, ids, _C.ROWS, task_rows, 1,
+             math.inf if limit is None else limit, table[:-16], None, None, act(T, K), act(slots, N),
+             act(slots, K), got)
     torch.cuda.synchronize()
     assert bool((table[-16:] == -1).all())
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))

@@ -102,9 +102,10 @@ TORCH_LIBRARY_PATH = os.path.join(PACKAGE, "libvllm_mi355x_torch.so")
 
 
 def build_torch_classes(verbose: bool = False) -> str:
-    """libvllm_mi355x_torch.so: the host-only torch custom classes the
-    reference's loader requires (csrc/torch_classes.cpp), built with g++
-    against the installed torch."""
+    """libvllm_mi355x_torch.so: the linear and MoE operators' implementations
+    (csrc/torch_ops.cpp) and the torch custom classes the reference's loader
+    requires (csrc/torch_classes.cpp): host-only, built with g++ against the
+    installed torch."""
     import torch
     from torch.utils import cpp_extension
 
@@ -113,10 +114,14 @@ def build_torch_classes(verbose: bool = False) -> str:
         raise RuntimeError("g++ not found (needed for libvllm_mi355x_torch.so)")
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
     cmd = [cxx, "-O2", "-fPIC", "-shared", "-std=c++17", "-w", f"-D_GLIBCXX_USE_CXX11_ABI={abi}"]
+    # (the HIP headers' platform, for torch's stream type)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cmd += ["-D__HIP_PLATFORM_AMD__=1", f"-I{os.path.join(rocm, 'include')}"]
     cmd += [f"-I{p}" for p in cpp_extension.include_paths()]
-    cmd += [os.path.join(CSRC, "torch_classes.cpp"), "-o", TORCH_LIBRARY_PATH + ".tmp"]
+    cmd += [os.path.join(CSRC, src) for src in ("torch_classes.cpp", "torch_ops.cpp")]
+    cmd += ["-o", TORCH_LIBRARY_PATH + ".tmp"]
     cmd += [f"-L{p}" for p in cpp_extension.library_paths()]
-    cmd += ["-lc10", "-ltorch_cpu", "-ltorch"]
+    cmd += ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"building libvllm_mi355x_torch.so failed:\n{res.stdout}\n{res.stderr}")

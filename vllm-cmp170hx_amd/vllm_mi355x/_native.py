@@ -13,8 +13,8 @@ import threading
 
 LIBRARY_NAME = "libvllm_mi355x.so"
 LIBRARY_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIBRARY_NAME)
-# The host-only torch custom classes the reference's loader requires
-# (csrc/torch_classes.cpp), loaded with torch.ops.load_library.
+# The host-only operator implementations (csrc/torch_ops.cpp) and the torch
+# custom classes the reference's loader requires (csrc/torch_classes.cpp).
 TORCH_CLASSES_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)),
                                   "libvllm_mi355x_torch.so")
 ABI_VERSION = 1
@@ -148,6 +148,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_torch_loaded = False
 _lock = threading.Lock()
 
 
@@ -178,6 +179,27 @@ def load() -> ctypes.CDLL:
             raise ImportError(f"{LIBRARY_NAME} ABI {version}, expected {ABI_VERSION}")
         _lib = lib
     return _lib
+
+
+def load_torch() -> None:
+    """Loads the operators' library and gives it load()'s entry points, once."""
+    global _torch_loaded
+    if _torch_loaded:
+        return
+    lib = load()
+    with _lock:
+        if _torch_loaded:
+            return
+        import torch
+        if not os.path.exists(TORCH_CLASSES_PATH):
+            raise ImportError(f"{TORCH_CLASSES_PATH} is not built: run "
+                              "python vllm-cmp170hx_amd/build.py")
+        torch.ops.load_library(TORCH_CLASSES_PATH)
+        bind = ctypes.CDLL(TORCH_CLASSES_PATH).vllm_mi355x_torch_bind
+        bind.argtypes, bind.restype = [c_vp], c_int
+        if bind(lib._handle):
+            raise ImportError(f"{LIBRARY_NAME} lacks an entry point of the operators")
+        _torch_loaded = True
 
 
 def last_error() -> str:

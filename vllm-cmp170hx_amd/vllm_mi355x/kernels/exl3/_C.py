@@ -1,21 +1,18 @@
 """The ``_exl3_C`` operator library on ROCm: the reference's schemas
 (csrc/exl3/module.cpp:12-67), each CUDA kernel implemented by a call into
 libvllm_mi355x.so with the tensors' device pointers on torch's current
-stream.  Tensor-level checks (device, dtype, contiguity, rank) are made here
-with the reference's messages (csrc/exl3/common.h:42-61, dense.cu:85-93);
-geometry, workspace and overlap checks are made by the native library.
+stream.  Tensor-level checks (device, dtype, contiguity, rank) are made with
+the reference's messages (csrc/exl3/common.h:42-61, dense.cu:85-93): those of
+the linear and MoE operators in C++ (csrc/torch_ops.cpp, with their
+implementations), the others' here; geometry, workspace and overlap checks are
+made by the native library.
 """
 
 from __future__ import annotations
 
-import os
-
 import torch
 
 from ... import _native
-
-_DTYPE_CODES = {torch.bfloat16: _native.BF16, torch.float16: _native.FP16,
-                torch.float32: _native.FP32}
 
 # Bumped with the reference's own meaning (module.cpp:86-88): 3 = moe_out_v2
 # takes bits_x2, 2 = the MoE operators take swiglu_limit.
@@ -118,34 +115,6 @@ def _stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def linear_out_impl(x, trellis, suh, svh, bits_x2, codebook, logical_in, logical_out, out,
-                    workspace) -> None:
-    if not x.is_cuda:
-        raise RuntimeError("EXL3 x must be CUDA")
-    _check_tensor(x, x, (torch.bfloat16, torch.float16), "x")
-    _check_tensor(trellis, x, (torch.int16,), "trellis")
-    _check_tensor(suh, x, (torch.float16,), "suh")
-    _check_tensor(svh, x, (torch.float16,), "svh")
-    if out.dtype not in (torch.bfloat16, torch.float16, torch.float32):
-        raise RuntimeError("EXL3 linear out must be BF16, FP16 or FP32")
-    _check_tensor(out, x, (out.dtype,), "out")
-    _check_tensor(workspace, x, (torch.float32,), "workspace")
-    if not (x.dim() == 2 and trellis.dim() == 3 and suh.dim() == 1 and svh.dim() == 1
-            and out.dim() == 2):
-        raise RuntimeError(
-            "EXL3 linear requires rank-2 x/out, rank-3 trellis and rank-1 scales")
-    lib = _native.load()
-    with torch.cuda.device(x.device):
-        status = lib.exl3_linear_out(
-            x.data_ptr(), _DTYPE_CODES[x.dtype], x.size(0), x.size(1),
-            trellis.data_ptr(), trellis.size(0), trellis.size(1), trellis.size(2),
-            suh.data_ptr(), suh.numel(), svh.data_ptr(), svh.numel(),
-            int(bits_x2), int(codebook), int(logical_in), int(logical_out),
-            out.data_ptr(), _DTYPE_CODES[out.dtype], out.size(0), out.size(1),
-            workspace.data_ptr(), workspace.numel(), _stream(x.device))
-    _native.check(status)
-
-
 def linear_workspace_size_impl(max_rows, padded_in, padded_out) -> int:
     size = _native.load().exl3_linear_workspace_size(max_rows, padded_in, padded_out)
     if size < 0:
@@ -175,91 +144,12 @@ def decode_impl(trellis, bits_x2, codebook, out) -> None:
     _native.check(status)
 
 
-def _check_integer(t, x, name):
-    if t.dtype not in (torch.int32, torch.int64):
-        raise RuntimeError(f"{name} must have int32 or int64 dtype")
-    _check_tensor(t, x, (t.dtype,), name)
-
-
-def _moe_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map, intermediate_size,
-              bits_x2, out, workspace, swiglu_limit) -> None:
-    """Checks of csrc/exl3/moe.cu:323-364, then the native operator."""
-    if not x.is_cuda:
-        raise RuntimeError("EXL3 x must be CUDA")
-    _check_tensor(x, x, (torch.bfloat16, torch.float16), "x")
-    _check_integer(topk_ids, x, "topk_ids")
-    _check_integer(expert_map, x, "expert_map")
-    _check_tensor(topk_weights, x, (torch.float32,), "topk_weights")
-    _check_tensor(packed_ptrs, x, (torch.int64,), "packed_ptrs")
-    _check_tensor(packed_meta, x, (torch.int64,), "packed_meta")
-    _check_tensor(out, x, (x.dtype,), "out")
-    _check_tensor(workspace, x, (torch.float32,), "workspace")
-    if not (x.dim() == 2 and out.dim() == 2 and topk_ids.dim() == 2 and topk_weights.dim() == 2
-            and expert_map.dim() == 1 and packed_ptrs.dim() == 3 and packed_meta.dim() == 3):
-        raise RuntimeError("EXL3 MoE tensor ranks mismatch")
-    rows, hidden = x.shape
-    if not (topk_ids.size(0) == rows and topk_weights.shape == topk_ids.shape
-            and out.shape == x.shape):
-        raise RuntimeError("EXL3 MoE row/topk/output geometry mismatch")
-    experts = packed_ptrs.size(0)
-    if not (packed_ptrs.size(1) == 3 and packed_ptrs.size(2) == 3 and packed_meta.size(0) == experts
-            and packed_meta.size(1) == 3 and packed_meta.size(2) == 4):
-        raise RuntimeError("EXL3 MoE pointer/metadata geometry mismatch")
-    lib = _native.load()
-    with torch.cuda.device(x.device):
-        status = lib.exl3_moe_out(
-            x.data_ptr(), _DTYPE_CODES[x.dtype], rows, hidden, topk_ids.data_ptr(),
-            int(topk_ids.dtype == torch.int64), topk_weights.data_ptr(), topk_ids.size(1),
-            packed_ptrs.data_ptr(), packed_meta.data_ptr(), experts, expert_map.data_ptr(),
-            int(expert_map.dtype == torch.int64), expert_map.numel(), int(intermediate_size),
-            int(bits_x2), out.data_ptr(), _DTYPE_CODES[out.dtype], workspace.data_ptr(),
-            workspace.numel(), float(swiglu_limit), _stream(x.device))
-    _native.check(status)
-
-
-def moe_out_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map,
-                 intermediate_size, out, workspace, swiglu_limit=0.0) -> None:
-    _moe_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map, intermediate_size,
-              0, out, workspace, swiglu_limit)
-
-
-# The one rate every routed matrix of a moe_out_prefill call has: the
-# reference's operator is built for bits_x2 10 with codebook 2 alone
-# (csrc/exl3/moe_prefill.cu:37-40, :169-171).
-MOE_PREFILL_BITS_X2 = 10
-
-
-def moe_out_prefill_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map,
-                         intermediate_size, out, workspace, swiglu_limit=0.0) -> None:
-    """moe_out's schema at the reference's prefill operator's one rate: the
-    fixed-rate path (tile GEMM for the experts with many routed rows, at
-    any hidden / intermediate size); an expert of another format gets NaN
-    rows where the reference's kernel traps."""
-    _moe_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map, intermediate_size,
-              MOE_PREFILL_BITS_X2, out, workspace, swiglu_limit)
-
-
-def moe_out_v2_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map,
-                    intermediate_size, bits_x2, out, workspace, swiglu_limit=0.0) -> None:
-    if int(bits_x2) <= 0:
-        raise RuntimeError("EXL3 MoE v2 needs the layer's bits_x2")
-    _moe_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map, intermediate_size,
-              bits_x2, out, workspace, swiglu_limit)
-
-
 def moe_workspace_size_impl(max_rows, hidden_size, intermediate_size, topk, local_experts) -> int:
     size = _native.load().exl3_moe_workspace_size(max_rows, hidden_size, intermediate_size, topk,
                                                   local_experts)
     if size < 0:
         raise RuntimeError(_native.last_error())
     return int(size)
-
-
-def moe_out_v2_mixed_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map,
-                          intermediate_size, bits_x2, out, workspace, swiglu_limit=0.0) -> None:
-    """The _mixed variants: every expert's own format, decoded at run time."""
-    _moe_impl(x, topk_ids, topk_weights, packed_ptrs, packed_meta, expert_map, intermediate_size,
-              0, out, workspace, swiglu_limit)
 
 
 def _ple_check(t, name, dtype, ndim, device) -> None:
@@ -349,29 +239,14 @@ def register() -> None:
     lib = torch.library.Library("_exl3_C", "DEF")
     for schema in SCHEMAS.values():
         lib.define(schema)
+    # the linear and MoE operators' implementations, and
     # torch.classes._exl3_C.PleHostReader / EngramHostFetch (stubs that raise)
-    if not os.path.exists(_native.TORCH_CLASSES_PATH):
-        raise ImportError(f"{_native.TORCH_CLASSES_PATH} is not built: run "
-                          "python vllm-cmp170hx_amd/build.py")
-    torch.ops.load_library(_native.TORCH_CLASSES_PATH)
-    lib.impl("linear_out", linear_out_impl, "CUDA")
-    lib.impl("linear_out_splitk", linear_out_impl, "CUDA")
+    _native.load_torch()
     lib.impl("exl3_decode", decode_impl, "CUDA")
-    lib.impl("moe_out", moe_out_impl, "CUDA")
-    lib.impl("moe_out_v2", moe_out_v2_impl, "CUDA")
     lib.impl("linear_workspace_size", linear_workspace_size_impl, "CompositeImplicitAutograd")
     lib.impl("moe_workspace_size", moe_workspace_size_impl, "CompositeImplicitAutograd")
     lib.impl("moe_workspace_size_v2", moe_workspace_size_impl, "CompositeImplicitAutograd")
     lib.impl("linear_splitk_splits", linear_splitk_splits_impl, "CompositeImplicitAutograd")
-    for name in _LINEAR_ALIASES:
-        lib.impl(name, linear_out_impl, "CUDA")
-    for name in _MOE_ALIASES:
-        lib.impl(name, moe_out_impl, "CUDA")
-    lib.impl("moe_out_prefill", moe_out_prefill_impl, "CUDA")
-    for name in _MOE_V2_ALIASES + _MOE_V2_TRY:
-        lib.impl(name, moe_out_v2_impl, "CUDA")
-    for name in _MOE_V2_MIXED:
-        lib.impl(name, moe_out_v2_mixed_impl, "CUDA")
     for name in _SIZE_ALIASES:
         lib.impl(name, moe_workspace_size_impl, "CompositeImplicitAutograd")
     lib.impl("ple_decode_out", ple_decode_out_impl, "CUDA")

@@ -252,6 +252,10 @@ def exl3_linear(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: 
         row_chunk = linear_row_chunk(suh.numel(), svh.numel())
     workspace = _linear_scratch(x.device)
     out = torch.empty((x.shape[0], logical_out), dtype=out_dtype, device=x.device)
+    if 0 < x.shape[0] <= row_chunk:
+        torch.ops._exl3_C.linear_out(x, trellis, suh, svh, bits_x2, codebook, x.shape[1],
+                                     logical_out, out, workspace)
+        return out
     for start in range(0, x.shape[0], row_chunk):
         linear_out(x[start:start + row_chunk], trellis, suh, svh, bits_x2, codebook,
                    x.shape[1], logical_out, out[start:start + row_chunk], workspace)

@@ -20,6 +20,9 @@ from ... import _native
 
 _DTYPE_CODES = {torch.bfloat16: _native.BF16, torch.float16: _native.FP16}
 
+# the launches of fused (csrc/torch_ops.cpp, marlin_moe)
+STAGED, DIRECT, ROWS, IDENTITY = 0, 1, 2, 3
+
 MODE_PARTIAL, MODE_STORE, MODE_TOPK, MODE_SWIGLU = 0, 1, 2, 3
 
 # build_info keys (ampere_marlin/module.cpp:9-15): abi_version 1, prefill
@@ -156,35 +159,16 @@ def rows_table(slots: int, experts: int, task_rows: int) -> int:
     return int(size)
 
 
-def rows(x, w1, s1, w2, s2, ids, topk_w, top_k, limit, task_rows, table, xp, h, c3) -> None:
-    """marlin_moe_rows on torch tensors: the slot rows c3 of moe_sum from x."""
-    K, N = x.size(1), h.size(1)
-    _require(x.dtype in _DTYPE_CODES and x.dim() == 2 and x.stride(1) == 1,
-             "a: bf16 or fp16, unit inner stride")
-    for w, s, k, n in ((w1, s1, K, 2 * N), (w2, s2, N, K)):
-        _require(s.dtype == x.dtype and w.dtype == torch.int32 and w.is_contiguous()
-                 and s.is_contiguous(), "weights contiguous, scales of the activation dtype")
-        _require(w.dim() == 3 and w.size(1) * 16 == k and w.size(2) == 2 * n,
-                 "w: int32 [E, K/16, 2N]")
-        _require(s.dim() == 3 and s.size(0) == w.size(0) and s.size(1) * 128 == k
-                 and s.size(2) == n, "s: [E, K/128, N]")
-    _require(ids.dtype == torch.int32 and ids.is_contiguous() and table.dtype == torch.int32,
-             "routing dtypes")
-    _require(topk_w.dtype == torch.float32 and topk_w.is_contiguous()
-             and topk_w.numel() == ids.numel() == x.size(0) * top_k, "topk weights fp32")
-    for t, rows_, cols in ((xp, x.size(0), K), (h, ids.numel(), N), (c3, ids.numel(), K)):
-        _require(t.dtype == x.dtype and t.is_contiguous() and tuple(t.shape) == (rows_, cols),
-                 "scratch rows of the activation dtype")
-    for t, name in ((w1, "w1"), (s1, "s1"), (w2, "w2"), (s2, "s2"), (ids, "ids"),
-                    (topk_w, "topk_w"), (table, "table"), (xp, "xp"), (h, "h"), (c3, "c3")):
-        _on(t, x.device, name)
-    with torch.cuda.device(x.device):
-        status = _native.load().marlin_moe_rows(
-            x.data_ptr(), _DTYPE_CODES[x.dtype], x.size(0), x.stride(0), w1.data_ptr(),
-            s1.data_ptr(), w2.data_ptr(), s2.data_ptr(), w1.size(0), ids.data_ptr(),
-            topk_w.data_ptr(), int(top_k), K, N, float(limit), int(task_rows), table.data_ptr(),
-            table.numel(), xp.data_ptr(), h.data_ptr(), c3.data_ptr(), _stream(x.device))
-    _native.check(status)
+def fused(x, w1, w2, s1, s2, topk_w, ids, path, block_size, ksplit, limit, lists, expert_ids, ntpp,
+          act, h, c3, out) -> None:
+    """Every launch of one fused call on one of the paths above: checks and
+    launches in one operator, on torch's current stream."""
+    if not x.is_cuda:
+        raise RuntimeError("tensors must be on the activation device")
+    _native.load_torch()
+    torch.ops._vllm_mi355x.marlin_moe.default(x, w1, w2, s1, s2, topk_w, ids, path, block_size,
+                                              ksplit, limit, lists, expert_ids, ntpp, act, h, c3,
+                                              out)
 
 
 def permute_act(a, out) -> None:
@@ -390,7 +374,7 @@ def register() -> None:
     global _library
     if _library is not None:
         return
-    _native.load()
+    _native.load_torch()
     lib = torch.library.Library("_ampere_marlin_C", "DEF")
     for schema in SCHEMAS.values():
         lib.define(schema)

@@ -22,7 +22,7 @@ import torch
 
 from . import _C
 from . import split_align as split_align_mod
-from ..moe.align import align_sizes, kernel_moe_align_block_size
+from ..moe.align import align_sizes
 from ..moe.routing import moe_sum
 
 
@@ -146,7 +146,7 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
     prefill.run, marlin_moe/prefill.py:381-447).  All give the same sums: a
     row's sums depend only on its own activations, expert and K split.  The
     automatic choice also takes row lists for calls with many rows per expert
-    (_rows_path; K split 1)."""
+    (marlin_moe_rows; K split 1)."""
     M, K = hidden_states.shape
     E = w1.size(0)
     N = w2.size(1) * 16
@@ -175,8 +175,13 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
     if path is None and block_size is None and ksplit is None and bs > _DIRECT_MAX_BLOCK:
         task_rows = rows_task_rows(hidden_states, w1, w2, w1_scale, w2_scale, topk)
         if task_rows:
-            return _rows_path(hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, local, out,
-                              limit, task_rows, workspace)
+            # the slots grouped by expert in tasks of task_rows rows, each
+            # task's weights dequantized once
+            shapes = {"table": (_C.rows_table(slots, E, task_rows),), "xp": (M, K),
+                      "h": (slots, N), "c3": (slots, K)}
+            _launch(_C.ROWS, hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, local,
+                    task_rows, 1, limit, shapes, workspace, out)
+            return out
     if path is None:
         direct = ksplit in (None, 1) and direct_applies(M, topk, K, N, E, bs)
     elif path == "split":
@@ -193,78 +198,31 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
     ks = 1 if direct else (ksplit or choose_w13_ksplit(blocks_est, 2 * N, K, bs))
     shapes = workspace_shapes(M, topk, K, N, E, bs, ks, direct)
     ws = workspace if workspace is not None else {}
-    buf = {}
+    # one token: its top-k slots route to distinct experts, so each slot is its
+    # own block (identity routing, no alignment launch)
+    kind = _C.DIRECT if direct else (_C.IDENTITY if M == 1 and path is None else _C.STAGED)
+    _launch(kind, hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, local, bs, ks, limit,
+            shapes, workspace, out)
+    return out
+
+
+def _launch(kind, hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, local, block_size, ksplit,
+            limit, shapes, workspace, out):
+    """The call's scratch, from the workspace where it is large enough, and its
+    launches (csrc/torch_ops.cpp)."""
+    ws = workspace if workspace is not None else {}
     for name, shape in shapes.items():
         dtype = {"part": torch.float32, "h": hidden_states.dtype, "xp": hidden_states.dtype,
                  "c3": hidden_states.dtype}.get(name, torch.int32)
         t = ws.get(name)
         numel = math.prod(shape)
         if t is None or t.numel() < numel or t.dtype != dtype:
-            t = torch.empty(numel, dtype=dtype, device=hidden_states.device)
-            ws[name] = t
-        buf[name] = t.view(-1)[:numel].view(shape)
-    tw = topk_weights.to(torch.float32).contiguous().view(-1)
-    if direct:
-        # the alignment and the w13 GEMM's k-permuted input in one launch
-        _C.align_permute(local, E, bs, buf["sorted"], buf["expert_ids"], buf["ntpp"], hidden_states,
-                         buf["xp"])
-        _C.gemm_direct(buf["xp"], w1, w1_scale, buf["sorted"], buf["expert_ids"], buf["ntpp"], None,
-                       topk, slots, K, 2 * N, bs, _C.MODE_SWIGLU, 1, limit, out=buf["h"])
-        _C.gemm_direct(buf["h"], w2, w2_scale, buf["sorted"], buf["expert_ids"], buf["ntpp"], tw, 1,
-                       slots, N, K, bs, _C.MODE_TOPK, 1, out=buf["c3"])
-        moe_sum(buf["c3"].view(M, topk, K), out, local, E)
-        return out
-    if M == 1 and path is None:
-        # one token: its top-k slots route to distinct experts, so each slot
-        # is its own block (identity routing, no alignment launch)
-        sorted_ids, expert_ids, ntpp = None, local.view(-1), None
-    else:
-        kernel_moe_align_block_size(local, E, bs, buf["sorted"], buf["expert_ids"], buf["ntpp"],
-                                    None, None)
-        sorted_ids, expert_ids, ntpp = buf["sorted"], buf["expert_ids"], buf["ntpp"]
-    if N % 64 == 0:
-        # the w13 partials and their SwiGLU in one launch
-        _C.w13_act(hidden_states, w1, w1_scale, sorted_ids, expert_ids, ntpp, local.view(-1),
-                   topk, slots, K, 2 * N, bs, ks, limit, buf["part"], buf["h"])
-    else:
-        _C.gemm(hidden_states, w1, w1_scale, sorted_ids, expert_ids, ntpp, None,
-                topk, slots, K, 2 * N, bs, _C.MODE_PARTIAL, ks, part=buf["part"])
-        _C.act(buf["part"], local.view(-1), ks, slots, N, limit, buf["h"])
-    if sorted_ids is None:
-        # identity routing: the w2 rows and their top-k sum in one launch
-        _C.w2_sum(buf["h"], w2, w2_scale, expert_ids, tw, topk, slots, N, K, bs, buf["c3"], out)
-        return out
-    _C.gemm(buf["h"], w2, w2_scale, sorted_ids, expert_ids, ntpp, tw, 1, slots,
-            N, K, bs, _C.MODE_TOPK, 1, out=buf["c3"])
-    moe_sum(buf["c3"].view(M, topk, K), out, local, E)
-    return out
-
-
-def _rows_path(hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, local, out, limit,
-               task_rows, workspace):
-    """Many rows per expert: the slots grouped by expert in tasks of task_rows
-    rows, each task's weights dequantized once (marlin_moe_rows)."""
-    M, K = hidden_states.shape
-    N, E = w2.size(1) * 16, w1.size(0)
-    topk = local.size(1)
-    slots = M * topk
-    ws = workspace if workspace is not None else {}
-    buf = {}
-    for name, shape, dtype in (("table", (_C.rows_table(slots, E, task_rows),), torch.int32),
-                               ("xp", (M, K), hidden_states.dtype),
-                               ("h", (slots, N), hidden_states.dtype),
-                               ("c3", (slots, K), hidden_states.dtype)):
-        t = ws.get(name)
-        numel = math.prod(shape)
-        if t is None or t.numel() < numel or t.dtype != dtype:
-            t = torch.empty(numel, dtype=dtype, device=hidden_states.device)
-            ws[name] = t
-        buf[name] = t.view(-1)[:numel].view(shape)
-    tw = topk_weights.to(torch.float32).contiguous().view(-1)
-    _C.rows(hidden_states, w1, w1_scale, w2, w2_scale, local, tw, topk, limit, task_rows,
-            buf["table"], buf["xp"], buf["h"], buf["c3"])
-    moe_sum(buf["c3"].view(M, topk, K), out, local, E)
-    return out
+            ws[name] = torch.empty(numel, dtype=dtype, device=hidden_states.device)
+    lists = (ws["table"], None, None) if kind == _C.ROWS else (
+        ws["sorted"], ws["expert_ids"], ws["ntpp"])
+    tw = topk_weights.to(torch.float32).contiguous()
+    _C.fused(hidden_states, w1, w2, w1_scale, w2_scale, tw, local, kind, block_size, ksplit, limit,
+             *lists, ws["xp" if "xp" in shapes else "part"], ws["h"], ws["c3"], out)
 
 
 def _split_path(hidden_states, w1, w2, w1_scale, w2_scale, topk_weights, local, out, limit, E,
