@@ -122,6 +122,27 @@ __device__ __forceinline__ float xor_lanes(float v, int lane) {
   return __builtin_bit_cast(float, r);
 }
 
+// The 4 x 4 dwords d[i] of a quad's lanes (lane & 3 = j) transposed: lane j's
+// d[i] becomes lane i's d[j] (two exchanges, by DPP quad permutes).  Every lane
+// of the quad must be active.
+__device__ __forceinline__ void quad_transpose(uint32_t (&d)[4], int lane) {
+  const bool odd = lane & 1, upper = lane & 2;
+#pragma unroll
+  for (int i = 0; i < 4; i += 2) {  // lane j's d[i | !j0] <-> lane (j ^ 1)'s d[i | j0]
+    const uint32_t a = uint32_t(__builtin_amdgcn_mov_dpp(int(d[i]), 0xB1, 0xF, 0xF, false));
+    const uint32_t b = uint32_t(__builtin_amdgcn_mov_dpp(int(d[i + 1]), 0xB1, 0xF, 0xF, false));
+    d[i] = odd ? b : d[i];
+    d[i + 1] = odd ? d[i + 1] : a;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t a = uint32_t(__builtin_amdgcn_mov_dpp(int(d[i]), 0x4E, 0xF, 0xF, false));
+    const uint32_t b = uint32_t(__builtin_amdgcn_mov_dpp(int(d[i + 2]), 0x4E, 0xF, 0xF, false));
+    d[i] = upper ? b : d[i];
+    d[i + 2] = upper ? d[i + 2] : a;
+  }
+}
+
 // A wavefront-uniform value the compiler cannot prove uniform (read through a
 // pointer into memory the kernel also writes, so with a vector load, or
 // derived from threadIdx.x / 64) moved to a scalar register: buffer

@@ -435,24 +435,30 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
 }
 
 // Writes inputs k0 .. k0 + 7 (k0 % 8 == 0) of t, scaled by the row's
-// power-of-two exponent, into the row's B-operand arrays: in b_order, inputs
-// 2i and 2i + 1 of the eight are adjacent halves (one dword store each) at
-// (k0 & ~31) + 8 i + 4 ((k0 >> 4) & 1) + 2 ((k0 >> 3) & 1).  The low parts
-// only when `lo` (rows of tile experts use the high parts alone).
+// power-of-two exponent, into the row's B-operand arrays.  A quad of lanes
+// holds a 32-input step (k0 & 31 = 8 (lane & 3)) and in b_order dword 4 i + j of
+// the step is inputs 2 i and 2 i + 1 of lane j, so the quad transposes its dwords
+// and each lane stores 16 consecutive bytes (a wavefront's 1 KB of high parts in
+// one instruction; with four dword stores of 16-byte pieces moe_form took 90 us
+// at 20480 rows of 2560, with these 76).  The low parts only when `lo` (rows of
+// tile experts use the high parts alone).
 __device__ __forceinline__ void store8(__amdgpu_buffer_rsrc_t dst, int kp, int k0, const float (&v)[8],
-                                       int e, bool lo) {
-  const int base = (k0 & ~31) + 4 * ((k0 >> 4) & 1) + 2 * ((k0 >> 3) & 1);
+                                       int e, bool lo, int lane) {
+  uint32_t hw[4], lw[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float t0 = ldexpf(v[2 * i], e);
     const float t1 = ldexpf(v[2 * i + 1], e);
     const _Float16 h0 = _Float16(t0), h1 = _Float16(t1);
     const _Float16 l0 = _Float16(t0 - float(h0)), l1 = _Float16(t1 - float(h1));
-    const uint32_t hw = uint32_t(__builtin_bit_cast(uint16_t, h0)) | (uint32_t(__builtin_bit_cast(uint16_t, h1)) << 16);
-    const uint32_t lw = uint32_t(__builtin_bit_cast(uint16_t, l0)) | (uint32_t(__builtin_bit_cast(uint16_t, l1)) << 16);
-    const int o = 2 * (base + 8 * i);  // bytes
-    __builtin_amdgcn_raw_buffer_store_b32(hw, dst, o, 0, 0);
-    if (lo) __builtin_amdgcn_raw_buffer_store_b32(lw, dst, o, 2 * kp, 0);
+    hw[i] = uint32_t(__builtin_bit_cast(uint16_t, h0)) | (uint32_t(__builtin_bit_cast(uint16_t, h1)) << 16);
+    lw[i] = uint32_t(__builtin_bit_cast(uint16_t, l0)) | (uint32_t(__builtin_bit_cast(uint16_t, l1)) << 16);
+  }
+  vq::quad_transpose(hw, lane);
+  __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{hw[0], hw[1], hw[2], hw[3]}, dst, 2 * k0, 0, 0);
+  if (lo) {
+    vq::quad_transpose(lw, lane);
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{lw[0], lw[1], lw[2], lw[3]}, dst, 2 * k0, 2 * kp, 0);
   }
 }
 
@@ -487,7 +493,7 @@ __global__ __launch_bounds__(256) void moe_form(Routing routing, const void* x, 
   const int z = int(blockIdx.y);  // gate and up in one launch: 0, 1
   const int projection = first_projection + z;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = vq::uniform(int(threadIdx.x >> 6));
   const int q = lane >> 4;   // the lane's block within a group
   const int l = lane & 15;   // its eight inputs within the block: 8 l ..
   const int64_t kp = kActivate ? lay.ipad : lay.hpad;
@@ -498,8 +504,12 @@ __global__ __launch_bounds__(256) void moe_form(Routing routing, const void* x, 
   const int g0 = kWaveRow ? 0 : wave;
   constexpr int kStride = kWaveRow ? 1 : 4;
   if (row >= table[0]) return;
-  const int64_t a = table[4 + row];
-  const int64_t e = reinterpret_cast<const int*>(ws + lay.ints())[lay.row_experts() + row];
+  // uniform() keeps the row, its expert and its pointers scalar: a buffer
+  // resource that the compiler takes to differ between lanes costs a loop over
+  // its values around each access (20480 rows of 2560: 76 us with those loops, 68
+  // without; 43 is the time of the writes alone)
+  const int64_t a = vq::uniform(table[4 + row]);
+  const int64_t e = vq::uniform(reinterpret_cast<const int*>(ws + lay.ints())[lay.row_experts() + row]);
   const int64_t* ptrs = routing.ptrs + e * 9;
   // the tile experts' rows (sorted rows from the first tile task's first
   // on) feed only the tile GEMM, which reads the low parts unless it runs
@@ -509,8 +519,8 @@ __global__ __launch_bounds__(256) void moe_form(Routing routing, const void* x, 
   int* exps = reinterpret_cast<int*>(ws + lay.ints()) + lay.exps() + a * (lay.kmax() / 128) + z;
   const __amdgpu_buffer_rsrc_t dst =
       make_rsrc(ws + (kActivate ? lay.act() : (z ? lay.input_up() : lay.input())) + a * kp, uint32_t(kp) * 4u);
-  const bool bad = routing.meta[e * 12 + projection * 4] != kp;
-  const uint16_t* suh = reinterpret_cast<const uint16_t*>(ptrs[projection * 3 + 1]);
+  const bool bad = vq::uniform(routing.meta[e * 12 + projection * 4]) != kp;
+  const uint16_t* suh = reinterpret_cast<const uint16_t*>(vq::uniform(ptrs[projection * 3 + 1]));
   // Buffer resources over the row's inputs (32-bit offsets; loads past the
   // end of x's row or of suh return zero, which forms zero).
   const int in_len = int(kActivate ? intermediate : hidden);
@@ -620,12 +630,12 @@ __global__ __launch_bounds__(256) void moe_form(Routing routing, const void* x, 
   }
 #pragma unroll
   for (int i = 0; i < kCache; ++i) {
-    if (g0 + kStride * i < groups && live(g0 + kStride * i)) store8(dst, int(kp), first_k(g0 + kStride * i), c[i], ex, lo);
+    if (g0 + kStride * i < groups && live(g0 + kStride * i)) store8(dst, int(kp), first_k(g0 + kStride * i), c[i], ex, lo, lane);
   }
   for (int64_t G = g0 + kStride * kCache; G < groups; G += kStride) {
     float v[8];
     form(G, v);
-    if (live(G)) store8(dst, int(kp), first_k(G), v, ex, lo);
+    if (live(G)) store8(dst, int(kp), first_k(G), v, ex, lo, lane);
   }
 }
 
