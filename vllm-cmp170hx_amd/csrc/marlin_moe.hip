@@ -264,7 +264,8 @@ __global__ __launch_bounds__(kThreads, 2) void marlin_gemm(GemmArgs g) {
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  // scalar: the weight loads' group offsets are built from it
+  const int wave = vq::uniform(tid >> 6);
   const int wk = wave % kWavesK;
   const int wt = wave / kWavesK;
   const int tile = int(blockIdx.x) * kTilesWG + wt;
