@@ -713,12 +713,18 @@ struct MoeGemvArgs {
   int64_t out_offset, out_step;
 };
 
-// LDS of a workgroup: two buffers of one 128-input block's B operands,
-// [buf][step][g][column][8 halves] (the epilogue's per-row sums reuse them:
-// kTaskRows x 128 floats), and the rows' exponents.
+// LDS of a workgroup: two buffers of the B operands of a stage, [buf][step][g]
+// [column][8 halves] (the epilogue's per-row sums reuse them: kTaskRows x 128
+// floats), and the rows' exponents.  A stage is four steps (128 inputs) of up to
+// 16 rows, two steps of up to 32: 16 KB either way, so that registers and not LDS
+// limit a CU's workgroups: five up to 4 bits (with 32 KB, four steps of 32 rows,
+// four).  64 tokens top-8 of 256 + 1 experts of 7168 / 2048 at 3 bits: 507 ->
+// 482 us a call; 200 tokens top-8 of 64 experts of 2048 / 768 at 3 and 4 bits: 156
+// -> 152.  Six workgroups spill (840 us), and six or seven with tasks of 16 rows
+// decode the larger experts twice (535).
 constexpr int kTaskCols = 2 * kTaskRows;
 struct MoeGemvShared {
-  _Float16 bop[2][4][4][kTaskCols][8];
+  _Float16 bop[8192];
   int rexp[kTaskRows];
 };
 static_assert(sizeof(MoeGemvShared::bop) >= sizeof(float) * kTaskRows * 128, "row sums fit the B staging");
@@ -741,11 +747,10 @@ __device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeG
   constexpr int kDepth = 4;
   constexpr int kRows = kTaskRows;
   constexpr int kSub = kRows / 8;
-  constexpr int kCols = kTaskCols;
-  constexpr int kChunks = kCols / 16;  // 16-byte B chunks per thread per block
+  constexpr int kChunks = 2;  // 16-byte B chunks per thread per stage, at most
   auto& bop = shared.bop;
   auto& rexp = shared.rexp;
-  float (*red)[128] = reinterpret_cast<float (*)[128]>(&bop[0][0][0][0][0]);
+  float (*red)[128] = reinterpret_cast<float (*)[128]>(&bop[0]);
 
   const int z = int(blockIdx.z);
   const int projection = args.projection + z;
@@ -801,44 +806,45 @@ __device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeG
   const int64_t row_bytes = tiles_n * tile_bytes;
   // (int: the host keeps the A x kp floats of a region below 2 GiB)
   const int steps = int(kp / 32);
-  const int kblocks = int(kp / 128);
   // the wavefront's two tiles of tile row 0
   const uint8_t* chunk = trellis + 2 * (4 * int64_t(blockIdx.x) + wave) * tile_bytes;
 
-  // B-operand staging of a block for the first kNs 8-row sub-blocks (kc =
+  // B-operand staging of kSteps steps for the first kNs 8-row sub-blocks (kc =
   // 16 kNs columns: rows 0 .. 8 kNs - 1, high and low parts): chunk c = tid +
-  // 256 i (i < kc / 16) is 16 bytes (step, g, column) = (c / (4 kc), c / kc
-  // % 4, c % kc), kept at that column of the kCols-wide LDS layout; columns
-  // of rows past the task read its last row again (their MFMA columns are
-  // never used).  Tasks of fewer rows stage (and read) fewer columns.
+  // 256 i is 16 bytes (step, g, column) = (c / (4 kc), c / kc % 4, c % kc);
+  // columns of rows past the task read its last row again (their MFMA columns
+  // are never used).  Tasks of fewer rows stage (and read) fewer columns.
   //    The B operands are read through a buffer over the input region
   //    (32-bit byte offsets: the region is A x kp floats, checked on the host).
   const __amdgpu_buffer_rsrc_t st_buf = __builtin_amdgcn_make_buffer_rsrc(
       ws + in_offset, 0, int(lay.assignments * kp * 4), 0x00020000);
+  auto stage_steps = [](auto ns_tag) { return std::integral_constant<int, decltype(ns_tag)::value <= 2 ? 4 : 2>{}; };
+  auto stage_chunks = [&](auto ns_tag) {
+    constexpr int n = decltype(stage_steps(ns_tag))::value * decltype(ns_tag)::value * 64 / 256;
+    static_assert(n >= 1 && n <= kChunks && 2 * n * 2048 <= int(sizeof(MoeGemvShared::bop) / sizeof(_Float16)), "stage");
+    return std::integral_constant<int, n>{};
+  };
   auto stage_offsets = [&](auto ns_tag, uint32_t (&off)[kChunks]) {
     constexpr int kc = 16 * decltype(ns_tag)::value;
 #pragma unroll
-    for (int i = 0; i < kc / 16; ++i) {
+    for (int i = 0; i < decltype(stage_chunks(ns_tag))::value; ++i) {
       const int c = tid + 256 * i;
       const int col = c % kc;
       const int64_t a = sorted[first + min(col >> 1, nrows - 1)];
       off[i] = uint32_t((a * 2 * kp + (col & 1) * kp + (c / (4 * kc)) * 32 + (c / kc % 4) * 8) * 2);
     }
   };
-  auto stage = [&](auto ns_tag, const uint32_t (&off)[kChunks], int kb, u32x4_t (&v)[kChunks]) {
-    constexpr int kc = 16 * decltype(ns_tag)::value;
+  auto stage = [&](auto ns_tag, const uint32_t (&off)[kChunks], int step, u32x4_t (&v)[kChunks]) {
 #pragma unroll
-    for (int i = 0; i < kc / 16; ++i) {
-      v[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(st_buf, int(off[i]),
-                                                                               int(kb * 256), 0));
+    for (int i = 0; i < decltype(stage_chunks(ns_tag))::value; ++i) {
+      v[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(st_buf, int(off[i]), step * 64, 0));
     }
   };
   auto put = [&](auto ns_tag, int buf, const u32x4_t (&v)[kChunks]) {
-    constexpr int kc = 16 * decltype(ns_tag)::value;
+    constexpr int n = decltype(stage_chunks(ns_tag))::value;
 #pragma unroll
-    for (int i = 0; i < kc / 16; ++i) {
-      const int c = tid + 256 * i;
-      *reinterpret_cast<u32x4_t*>(&bop[buf][c / (4 * kc)][c / kc % 4][c % kc][0]) = v[i];
+    for (int i = 0; i < n; ++i) {
+      *reinterpret_cast<u32x4_t*>(&bop[(buf * n * 256 + tid + 256 * i) * 8]) = v[i];
     }
   };
   if (tid < kRows) {
@@ -901,6 +907,8 @@ __device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeG
 
   auto stream = [&](auto aligned_tag, auto ns_tag) {
     constexpr int kNs = decltype(ns_tag)::value;  // sub-blocks staged and read
+    constexpr int kSteps = decltype(stage_steps(ns_tag))::value;
+    constexpr int kc = 16 * kNs;
     uint32_t st_off[kChunks];
     stage_offsets(ns_tag, st_off);
     // prologue: block 0's B operands, the first kDepth steps of trellis
@@ -912,19 +920,16 @@ __device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeG
     __syncthreads();
 
     // one 128-input block (4 steps) per iteration, branch-free around the
-    // loads: the last block re-stages itself into the buffer no step reads
+    // loads: the last stage re-stages itself into the buffer no step reads
     // again, and the trellis loads past the end reload the last step
     for (int s0 = 0; s0 < steps; s0 += kDepth) {
   #pragma unroll
       for (int i = 0; i < kDepth; ++i) {
         const int s = s0 + i;
         {
-          const int kb = s >> 2;
-          const int buf = int(kb & 1);
-          if (i == 0) {
-            progress_priority(s, steps);
-            stage(ns_tag, st_off, min(kb + 1, kblocks - 1), sv);
-          }
+          const int buf = int(s / kSteps & 1);
+          if (i == 0) progress_priority(s, steps);
+          if (i % kSteps == 0) stage(ns_tag, st_off, min(s + kSteps, steps - kSteps), sv);
           uint32_t q0[4], q1[4];
           if constexpr (kFixed) {
             uint32_t w0[kWords], w1[kWords];
@@ -953,7 +958,9 @@ __device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeG
           // then the MFMAs of the task's sub-blocks
           half8_t b[kSub];
   #pragma unroll
-          for (int sb = 0; sb < kNs; ++sb) b[sb] = *reinterpret_cast<const half8_t*>(&bop[buf][s & 3][g][16 * sb + m][0]);
+          for (int sb = 0; sb < kNs; ++sb) {
+            b[sb] = *reinterpret_cast<const half8_t*>(&bop[(((buf * kSteps + i % kSteps) * 4 + g) * kc + 16 * sb + m) * 8]);
+          }
   #pragma unroll
           for (int sb = 0; sb < kNs; ++sb) {
             if (sb < nsub) {
@@ -961,7 +968,7 @@ __device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeG
               acc2[sb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a2), b[sb], acc2[sb], 0, 0, 0);
             }
           }
-          if (i == 3) {
+          if (i % kSteps == kSteps - 1) {
             put(ns_tag, buf ^ 1, sv);
             __syncthreads();
           }
