@@ -514,8 +514,8 @@ def gpu_exl3_moe_prefill(torch, tokens=(2048, 65, 512, 3460), experts=256, hidde
     intermediate 640, every matrix bits_x2 10 mul1, top-10 from softmax of
     ~N(0, 1) logits, bf16 activations, 65 to 3460 rows, through
     _exl3_C::moe_out_prefill; the same 2048-row call through moe_out (the
-    run-time-format GEMV in 8-row tasks, what moe_out_prefill ran before it
-    had a many-row kernel) for comparison.  The first count is the line's
+    GEMV of a layer with a rate for every matrix, in 32-row tasks, no tile
+    GEMM) for comparison.  The first count is the line's
     headline."""
     from vllm_mi355x.kernels.exl3 import ops
 
@@ -574,7 +574,7 @@ def gpu_exl3_moe_prefill(torch, tokens=(2048, 65, 512, 3460), experts=256, hidde
             "precision": "fp16 hi+lo activations", **head, "by_tokens": by_tokens,
             "fp16_only": {"precision": "tile GEMM on fp16 activations (high parts alone)",
                           "by_tokens": fp16_only},
-            "runtime_decode_gemv": {"op": "moe_out (run-time-format GEMV, 8-row tasks)",
+            "runtime_decode_gemv": {"op": "moe_out (GEMV of any rate per matrix, 32-row tasks)",
                                     **runtime_gemv,
                                     "speedup_of_moe_out_prefill": round(
                                         runtime_gemv["us_per_forward"] / head["us_per_forward"], 2)}}

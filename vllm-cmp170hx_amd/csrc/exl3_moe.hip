@@ -8,7 +8,8 @@
 //     rows) and cuts each expert's rows into tasks of at most 32 rows: one workgroup
 //     below 8192 routed slots, else moe_route_count / moe_route /
 //     moe_route_fill over many workgroups.
-//  2. per projection (gate, up): moe_form builds t = H128(x[a / topk] * suh)
+//  2. per projection (gate and up together in calls of fewer than 8192 routed
+//     slots of at least 1024 inputs): moe_form builds t = H128(x[a / topk] * suh)
 //     of every local assignment, as FP16 high/low parts in MFMA B-operand
 //     order with one power-of-two scale per assignment row (the high parts
 //     alone for the tile experts' rows when the tile GEMM runs at FP16

@@ -67,11 +67,12 @@ def workspace_shapes(tokens: int, topk: int, hidden: int, inter: int, experts: i
 # hold more rows than that (over 22 on average, choose_block_size) run on row
 # lists (marlin_moe_rows), whose tasks hold up to 128 rows per dequantized weight.
 # Both sides measured, us per call in BF16 / FP16, 128 experts of 2048 / 768 at
-# top-8: 16 rows an expert, direct 130 / 93, rows 141 / 114; 25 rows, staged blocks
-# of 64 (what such calls ran on) 166 / 140, rows 142 / 118; 128 rows 442 / 376 and
-# 292 / 262.  Tasks of 128 rows were the best or within 5% of it from 25 to 512
-# rows an expert (64: 340 / 285 at 128 rows) but for 16 experts of 128 rows (96: 173
-# against 202).
+# top-8: 16 rows an expert, direct 118 / 92, rows 135 / 113; 25 rows, staged blocks
+# of 64 (what such calls ran on) 157 / 138, rows 132 / 118; 128 rows 415 / 362 and
+# 277 / 246.  Of tasks of 32 to 128 rows, 128 was the best or within a few percent
+# from 32 to 400 rows an expert, but where few experts hold about 128 rows each and
+# half of them need a second task (16 experts of 4096 / 1536, 128 rows: 190, in
+# tasks of 96 166; at 100 rows 138 against 162, at 200 205 against 251).
 _DIRECT_MAX_BLOCK = 32
 _TASK_ROWS = 128
 
