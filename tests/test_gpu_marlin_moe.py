@@ -635,3 +635,32 @@ def test_many_rows_per_expert_match_oracle(mm, device, dtype, limit, T):
     assert "table" in ws  # the row path ran
     expected = M.moe(x, dtype, ids, w, *layer.host, limit=math.inf if limit is None else limit)
     assert_close(host_bits(out), expected, dtype, f"many rows T={T}")
+
+
+@pytest.mark.parametrize("T", [1, 3, 40, 60])
+def test_fused_call_on_a_side_stream_and_its_refusals(mm, device, T):
+    """One operator issues a call's launches (identity, staged, direct and row
+    lists by T): a call on another stream, with inputs that require gradients,
+    equals the default stream's; wrong buffers are refused before any launch."""
+    print(f"fused operator T={T}", flush=True)
+    rng = np.random.default_rng(T)
+    E, K, N, topk = 4, 256, 128, 2
+    layer = Layer(rng, E, K, N, M.BF16, device)
+    x = dev_act(from_f32(rng.standard_normal((T, K)), M.BF16), M.BF16, device)
+    ids = dev(np.argsort(rng.random((T, E)), axis=1)[:, :topk].astype(np.int32), device)
+    w = dev(rng.random((T, topk)).astype(np.float32), device)
+    args = (layer.w1, layer.w2, layer.s1, layer.s2, w, ids)
+    want = mm[0].fused_marlin_moe(x, *args)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = mm[0].fused_marlin_moe(x.clone().requires_grad_(), *args)
+    side.synchronize()
+    assert not got.requires_grad
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for bad in ({"h": torch.empty(2 * T * topk, N, dtype=x.dtype, device=device)[::2]},
+                {"c3": torch.empty(T * topk, K, dtype=x.dtype)}):
+        with pytest.raises(RuntimeError):
+            mm[0].fused_marlin_moe(x, *args, workspace=dict(bad))
+    with pytest.raises(RuntimeError):
+        mm[0].fused_marlin_moe(x.cpu(), *args)
