@@ -65,15 +65,17 @@ int64_t exl3_linear_workspace_size(int64_t max_rows, int64_t padded_in, int64_t 
  * exl3_linear_out without a workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid allocation).  No counterpart in the
- * reference.  The same checks, kernels and results as exl3_linear_out; the
- * K-split partials (rows <= 32, in column ranges that fit) or the large-M
- * activations live in a static 16 MiB device array of the library (one per
+ * reference.  The same checks, kernels and results as exl3_linear_out with
+ * a workspace of 4M floats; the small-M path's K-split partials (in column
+ * ranges that fit) or the tile GEMM's activations and partial sums live in a
+ * static 16 MiB device array of the library (one per
  * device, held until the process ends; its address is looked up on the
  * first call on each device).  Calls of more than 32 rows need rows *
  * (padded_in + 1) floats of it: larger ones are rejected with an error
  * (exl3_linear_scratch_rows gives the limit).  Calls on one device share
  * the array: calls that overlap in time on one GPU (different streams)
- * race and must be ordered by the caller.  Allocates nothing.
+ * race and must be ordered by the caller; host threads that call on one
+ * stream need no lock (as for exl3_linear_out).  Allocates nothing.
  */
 int exl3_linear_out_scratch(const void* x, int x_dtype, int64_t rows, int64_t x_cols,
                             const void* trellis, int64_t tiles_k, int64_t tiles_n,
@@ -112,6 +114,10 @@ int exl3_linear_prefill_rows(void);
  *   out      [rows][logical_out] of out_dtype (VQ_BF16, VQ_FP16 or VQ_FP32)
  *   workspace FP32, exl3_linear_workspace_size(rows, ...) elements (or
  *            fewer, see there), 16-byte aligned, overlapping no other argument.
+ *            A call's launches pass data through it: calls that share one
+ *            must be on one stream, where they may come from several host
+ *            threads (a call's launches are issued under a lock of its
+ *            workspace's address).
  * The weights are decoded bit-exactly; the products are summed in FP32 on
  * the matrix cores, with the activations split into FP16 high and low
  * parts (about 22 significant bits, the activation precision of the

@@ -606,3 +606,38 @@ def test_tile_splits_match_oracle(ops, device, shape, bits_x2, codebook):
     want = O.linear_out(x, code, trellis, suh, svh, bits_x2, codebook, n - 3, O.FP32)
     for g in got:
         _assert_fp32_close(g, want, f"{shape}")
+
+
+def test_threads_on_one_stream_share_the_scratch(ops, device):
+    """exl3_linear keeps one scratch per stream, through which a call's launches
+    pass activations and partial sums: calls of several host threads on one
+    stream (8 rows: one launch; 20 and 40: three) must each give what they
+    give alone, bit for bit."""
+    import threading
+    print("threads on one stream", flush=True)
+    rng = np.random.default_rng(11)
+    k, n, bits_x2, codebook = 1152, 384, 8, 2
+    trellis, suh, svh = (_dev(a, device) for a in random_matrix(rng, k, n, bits_x2))
+    inputs = [_dev(random_acts(rng, rows, k, "fp16")[0], device) for rows in (20, 40, 20, 8)]
+
+    def call(x):
+        return ops.exl3_linear(x, trellis, suh, svh, bits_x2, codebook, n, out_dtype=torch.float32)
+
+    want = [call(x) for x in inputs]
+    torch.cuda.synchronize()
+    results = [[] for _ in inputs]
+    start = threading.Barrier(len(inputs))
+
+    def work(i):
+        start.wait()
+        for _ in range(200):
+            results[i].append(call(inputs[i]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(inputs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for got, w in zip(results, want):
+        assert len(got) == 200 and all(torch.equal(g, w) for g in got)

@@ -351,6 +351,18 @@ int check_linear(const void* x, int x_dtype, int64_t rows, int64_t x_cols, const
   return kOk;
 }
 
+// Held by a host thread while it issues a call's launches.  A call hands its
+// activations and partial sums from one launch to the next through its
+// workspace, so the launches of two calls that share a stream and a workspace
+// (several threads in exl3_linear, whose scratch is one per stream, or on
+// the static scratch) must follow one another call by call.  One of a few
+// mutexes, by the workspace's address: two workspaces that share one only
+// wait a launch's time for each other, and a call takes no second one.
+std::mutex& issue_mutex(const void* workspace) {
+  static std::mutex mutexes[64];
+  return mutexes[(uint64_t(reinterpret_cast<uintptr_t>(workspace)) >> 4) * 0x9E3779B97F4A7C15ull >> 58];
+}
+
 // The small-M path (chunks of kMaxGemvRows rows) with `partial`
 // holding `partial_numel` floats for the K-split partials.  A chunk whose
 // partials do not fit runs in column ranges (whole 128-column blocks) that
@@ -436,6 +448,7 @@ extern "C" int exl3_linear_out(const void* x, int x_dtype, int64_t rows, int64_t
   }
   if (rows == 0) return vq::kOk;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  const std::lock_guard<std::mutex> issuing(exl3::issue_mutex(workspace));
   if (rows > exl3::kGemvChunkedRows ||
       exl3::tile_small(rows, trellis, tiles_k, tiles_n, bits_x2, workspace_numel)) {
     return exl3::prefill_linear(x, x_dtype, rows, static_cast<const uint8_t*>(trellis), tiles_k,
@@ -516,6 +529,7 @@ extern "C" int exl3_linear_out_scratch(const void* x, int x_dtype, int64_t rows,
   float* scratch = exl3::scratch_address();
   if (!scratch) return vq::kHipFailure;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  const std::lock_guard<std::mutex> issuing(exl3::issue_mutex(scratch));
   if (rows > exl3::kGemvChunkedRows ||
       exl3::tile_small(rows, trellis, tiles_k, tiles_n, bits_x2, exl3::kScratchFloats)) {
     return exl3::prefill_linear(x, x_dtype, rows, static_cast<const uint8_t*>(trellis), tiles_k,
