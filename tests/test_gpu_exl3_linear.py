@@ -641,3 +641,39 @@ def test_threads_on_one_stream_share_the_scratch(ops, device):
     torch.cuda.synchronize()
     for got, w in zip(results, want):
         assert len(got) == 200 and all(torch.equal(g, w) for g in got)
+
+
+def _linear64(ops, x, trellis, suh, svh, bits_x2, codebook):
+    """H128(H128(x * suh) W) * svh in float64, W the decoded weights."""
+    h = torch.ones(1, 1, dtype=torch.float64, device=x.device)
+    while h.shape[0] < 128:
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
+    h /= 128 ** 0.5
+    t = ((x.double() * suh.double()).view(-1, 128) @ h).view(x.shape[0], -1)
+    y = t @ ops.decode(trellis, bits_x2, codebook).double()
+    return (y.view(-1, 128) @ h).view(x.shape[0], -1) * svh.double()
+
+
+# three, sixteen and one K split
+@pytest.mark.parametrize("k,n", [(1152, 384), (4096, 512), (2048, 65792)])
+def test_tile_sums_of_few_rows_are_as_exact_as_the_small_kernels(ops, device, prefill_switches, k, n):
+    """Calls of 17 to 32 rows run on either kernel (the small-M one in chunks
+    of 8 rows where the tile GEMM does not apply): the tile GEMM's error
+    against float64 is no larger.  Both errors are rms values over at least
+    12288 outputs, so their ratio is known to about 2%: bar 1.05 (with high and
+    low parts in one chain over a split's inputs it was 1.2 to 2.5)."""
+    print(f"few-row sums {k}x{n}", flush=True)
+    rng = np.random.default_rng(k + n)
+    bits_x2, codebook, rows = 4, 2, 32
+    trellis, suh, svh = (_dev(a, device) for a in random_matrix(rng, k, n, bits_x2))
+    x = _dev(random_acts(rng, rows, k, "fp16")[0], device)
+    want = _linear64(ops, x, trellis, suh, svh, bits_x2, codebook)
+    ws = torch.empty(ops.linear_workspace_size(rows, k, n), dtype=torch.float32, device=device)
+    errors = []
+    for kernel in (0, 1):  # tile GEMM, small-M chunks
+        prefill_switches[0](kernel)
+        out = torch.empty(rows, n, dtype=torch.float32, device=device)
+        ops.linear_out(x, trellis, suh, svh, bits_x2, codebook, k, n, out, ws)
+        errors.append(float((out.double() - want).pow(2).mean().sqrt()))
+    print(f"rms error: tile GEMM {errors[0]:.3g}, chunks {errors[1]:.3g}", flush=True)
+    assert errors[0] <= 1.05 * errors[1]

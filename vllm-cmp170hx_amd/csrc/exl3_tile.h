@@ -155,18 +155,29 @@ constexpr int tile_lds_bytes(int blocks, int parts, int bits_x2) {
   return kTileABufs * parts * blocks * 1024 + kTileWaves * kTileRing * tile_slot_bytes(bits_x2);
 }
 constexpr int tile_occupancy(int blocks, int bits_x2) {
-  const int registers = blocks <= 2 ? 4 : (blocks <= 4 ? 3 : 2);
+  const int registers = blocks == 4 ? 3 : 2;
   const int lds = 160 * 1024 / tile_lds_bytes(blocks, 2, bits_x2);
   return registers < lds ? registers : lds;
 }
 
 // kBlocks: the tile's 16-row blocks: 8 (up to 128 rows), or 2 and 4 for dense
-// calls of up to 32 and 64 rows, whose smaller accumulators and activation
-// tiles leave room for more wavefronts per SIMD.  At 2 row blocks a wavefront
+// calls of up to 32 and 64 rows.  At 2 row blocks a wavefront
 // and step take 0.43 us (900 cycles: the decode's 126 VALU instructions and 16
 // MFMAs, which share the SIMD's issue and add up) whether one or four
 // wavefronts share a SIMD; loads 5 to 8 steps ahead instead of 2 to 4
 // changed nothing.
+//
+// At 2 row blocks (calls of 9 to 32 rows, which the small-M kernel also
+// takes, in chunks) the FP32 sums are as short-chained as the small-M kernel's,
+// whose workgroups hold 4 to 32 steps: the high parts' products are
+// added over 4 steps, those sums over 16 steps, and those over the K range; the
+// low parts', 2^-11 of the high ones, in a chain of their own.  FP32 outputs'
+// error against 64 bits (2-norms), in 1e-7, the small-M kernel / these sums / one
+// chain of high and low parts: 1.69 / 1.53 / 2.42 at 4096 x 14336, 2.40 / 1.57 / 4.27 at
+// 8192 x 28672, 2.38 / 1.55 / 5.88 at 4096 x 151936, 1.48 / 1.49 / 1.94 at 1024 x
+// 1024.  The sums take 200 registers instead of 108 (two workgroups a CU, as
+// many as the splits make) and no time: 28.9 us at 20 rows of 4096 x 14336 with
+// either, 158 at 4096 x 151936.
 template <int kBitsX2, int kCodebook, bool kMoe, bool kLo, int kBlocks>
 __global__ __launch_bounds__(kTileThreads, tile_occupancy(kBlocks, kBitsX2)) void tile_gemm(TileArgs a) {
   constexpr int kRows = 16 * kBlocks;
@@ -344,7 +355,11 @@ __global__ __launch_bounds__(kTileThreads, tile_occupancy(kBlocks, kBitsX2)) voi
     }
   };
 
+  constexpr bool kShortChains = !kMoe && kLo && kBlocks == 2;
+  constexpr int kSums = kShortChains ? kBlocks : 1;
   f32x4_t acc[kBlocks][2][2];
+  f32x4_t low[kSums][2][2];               // short chains: the low parts' products
+  f32x4_t sum[kSums][2][2], total[kSums][2][2];  // high parts: over 16 steps, over the K range
 #pragma unroll
   for (int rb = 0; rb < kBlocks; ++rb)
 #pragma unroll
@@ -431,13 +446,16 @@ __global__ __launch_bounds__(kTileThreads, tile_occupancy(kBlocks, kBitsX2)) voi
       for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          acc[rb][p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[rb], b_cur[p][j], acc[rb][p][j], 0, 0, 0);
+          acc[rb][p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              ah[rb], b_cur[p][j], kShortChains && kS == 0 ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : acc[rb][p][j], 0, 0, 0);
       if constexpr (kLo) {
 #pragma unroll
         for (int p = 0; p < 2; ++p)
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[rb][p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[rb], b_cur[p][j], acc[rb][p][j], 0, 0, 0);
+          for (int j = 0; j < 2; ++j) {
+            f32x4_t& c = kShortChains ? low[kShortChains ? rb : 0][p][j] : acc[rb][p][j];
+            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[rb], b_cur[p][j], c, 0, 0, 0);
+          }
       }
     });
 #pragma unroll
@@ -456,11 +474,38 @@ __global__ __launch_bounds__(kTileThreads, tile_occupancy(kBlocks, kBitsX2)) voi
   // runs the loop of its height rounded up to 2, 4, 5, 6 or 8 row blocks (3
   // or 4 in a four-block tile).  None branches around an MFMA.
   auto run = [&](auto row_blocks) __attribute__((always_inline)) {
-    for (int s = 0; s < steps; s += kTileRing) {
+    auto four_steps = [&](int s) __attribute__((always_inline)) {
       step(s, std::integral_constant<int, 0>{}, row_blocks);
       step(s + 1, std::integral_constant<int, 1>{}, row_blocks);
       step(s + 2, std::integral_constant<int, 2>{}, row_blocks);
       step(s + 3, std::integral_constant<int, 3>{}, row_blocks);
+    };
+    if constexpr (kShortChains) {
+      auto each = [&](auto&& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rb = 0; rb < kBlocks; ++rb)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            f(rb, p, 0);
+            f(rb, p, 1);
+          }
+      };
+      const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+      each([&](int rb, int p, int j) { low[rb][p][j] = sum[rb][p][j] = total[rb][p][j] = zero; });
+      for (int s = 0; s < steps;) {
+        const int end = min(s + 4 * kTileRing, steps);
+        for (; s < end; s += kTileRing) {
+          four_steps(s);
+          each([&](int rb, int p, int j) { sum[rb][p][j] += acc[rb][p][j]; });
+        }
+        each([&](int rb, int p, int j) {
+          total[rb][p][j] += sum[rb][p][j];
+          sum[rb][p][j] = zero;
+        });
+      }
+      each([&](int rb, int p, int j) { acc[rb][p][j] = total[rb][p][j] + low[rb][p][j]; });
+    } else {
+      for (int s = 0; s < steps; s += kTileRing) four_steps(s);
     }
   };
   // A wavefront whose tile columns all lie past the matrix (in the last
