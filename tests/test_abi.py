@@ -91,6 +91,25 @@ def test_block_size_and_split_choice():
     assert 1 <= ks and (2048 // 128) % ks == 0 and (2048 // 128) // ks >= 4
 
 
+@pytest.mark.parametrize("experts,routed,hidden,inter,rows,want", [
+    # few workgroups with a long K: the staged path splits it
+    (8, 8, 14336, 512, 24, False), (8, 8, 14336, 512, 128, False), (2, 2, 7168, 256, 100, False),
+    (16, 16, 7168, 512, 24, False), (8, 8, 7168, 2048, 24, False), (32, 32, 14336, 512, 64, False),
+    (64, 64, 8192, 256, 48, False), (16, 16, 6144, 1024, 24, False),
+    # short K, enough workgroups, or enough rows for them
+    (8, 8, 4096, 1024, 24, True), (128, 128, 2048, 768, 24, True), (8, 8, 7168, 2048, 64, True),
+    (32, 32, 14336, 512, 128, True), (64, 64, 7168, 512, 24, True), (8, 8, 7168, 4096, 24, True),
+    # an eighth of the layer's experts held here: 24 rows a held expert's
+    # share of the slots are 3 routed ones
+    (16, 128, 2048, 768, 24, False), (4, 32, 4096, 1536, 64, False), (16, 128, 2048, 768, 200, True)])
+def test_row_lists_where_they_are_faster(experts, routed, hidden, inter, rows, want):
+    """The many-rows path of the fused Marlin MoE at the sizes where it was
+    measured against the staged path: chosen only where it is the faster one."""
+    from vllm_mi355x.kernels.marlin_moe.fused import rows_applies
+    topk = 2
+    assert rows_applies(rows * experts // topk, topk, hidden, inter, experts, routed) == want
+
+
 def test_linear_row_chunk_reaches_the_prefill_gemm():
     """The reference's fixed 8M-float dense scratch (ops.py:31-33) holds
     more rows per chunk than the small-M threshold at the prefill shapes,

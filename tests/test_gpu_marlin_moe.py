@@ -664,3 +664,27 @@ def test_fused_call_on_a_side_stream_and_its_refusals(mm, device, T):
             mm[0].fused_marlin_moe(x, *args, workspace=dict(bad))
     with pytest.raises(RuntimeError):
         mm[0].fused_marlin_moe(x.cpu(), *args)
+
+
+@pytest.mark.parametrize("K,N,held,want", [(256, 128, 4, "table"), (256, 128, 32, "part"),
+                                           (7168, 128, 4, "part")])
+def test_many_rows_run_where_row_lists_are_faster(mm, device, K, N, held, want):
+    """92 slots over 4 experts: row lists; the same slots over a map of 32
+    experts (about 3 routed rows a held expert), or a long K in few
+    workgroups: the staged path, on its own buffers."""
+    print(f"row lists or staged K={K} N={N} held 4 of {held}", flush=True)
+    rng = np.random.default_rng(K + held)
+    E, T, topk, dtype = 4, 46, 2, M.BF16
+    layer = Layer(rng, E, K, N, dtype, device)
+    ids, w = routing(rng, T, held, topk)
+    emap = np.full(held, -1, np.int32)
+    emap[:E] = np.arange(E)
+    x = from_f32(rng.standard_normal((T, K)), dtype)
+    ws = {}
+    out = mm[0].fused_marlin_moe(dev_act(x, dtype, device), layer.w1, layer.w2, layer.s1, layer.s2,
+                                 dev(w, device), dev(ids, device), workspace=ws,
+                                 expert_map=dev(emap, device) if held > E else None)
+    torch.cuda.synchronize()
+    assert want in ws and not {"table", "part"} - {want} & set(ws)
+    expected = M.moe(x, dtype, emap[ids], w, *layer.host)
+    assert_close(host_bits(out), expected, dtype, f"K={K} held={held}")

@@ -67,12 +67,12 @@ def workspace_shapes(tokens: int, topk: int, hidden: int, inter: int, experts: i
 # hold more rows than that (over 22 on average, choose_block_size) run on row
 # lists (marlin_moe_rows), whose tasks hold up to 128 rows per dequantized weight.
 # Both sides measured, us per call in BF16 / FP16, 128 experts of 2048 / 768 at
-# top-8: 16 rows an expert, direct 118 / 92, rows 135 / 113; 25 rows, staged blocks
-# of 64 (what such calls ran on) 157 / 138, rows 132 / 118; 128 rows 415 / 362 and
-# 277 / 246.  Of tasks of 32 to 128 rows, 128 was the best or within a few percent
+# top-8: 16 rows an expert, direct 118 / 92, rows 135 / 113; 24 rows, staged blocks
+# of 64 (what such calls ran on) 155 / 130, rows 137 / 116; 128 rows 413 / 370 and
+# 289 / 262.  Of tasks of 32 to 128 rows, 128 was the best or within a few percent
 # from 32 to 400 rows an expert, but where few experts hold about 128 rows each and
 # half of them need a second task (16 experts of 4096 / 1536, 128 rows: 190, in
-# tasks of 96 166; at 100 rows 138 against 162, at 200 205 against 251).
+# tasks of 96 166, staged 210; at 100 rows 138 against 162, at 200 205 against 251).
 _DIRECT_MAX_BLOCK = 32
 _TASK_ROWS = 128
 
@@ -94,10 +94,44 @@ def direct_applies(tokens: int, topk: int, hidden: int, inter: int, experts: int
     return touched * (2 * inter // 256) >= _DIRECT_MIN_WORKGROUPS
 
 
+# Hidden sizes up to which row lists win whatever the experts' number, and the
+# w13 workgroups above it (rows_applies).
+_ROWS_ANY_HIDDEN = 4096
+_ROWS_MIN_WORKGROUPS = 128
+_ROWS_FULL_WORKGROUPS = 256
+_ROWS_FULL_HIDDEN = 7168
+
+
+def rows_applies(tokens: int, topk: int, hidden: int, inter: int, experts: int,
+                 routed_experts: int) -> bool:
+    """Whether row lists are faster than the staged blocks of 64 for a call of
+    over 22 rows per routed expert (routed_experts: those of the whole layer;
+    experts: those held here, which run their share of the rows).
+
+    A workgroup of the row lists runs the whole K range of up to 128 rows; the
+    staged w13 splits K until the chip is full.  So few workgroups and a long K
+    are the staged path's.  Measured, row lists' time over the staged path's:
+    0.42 to 0.98 over 1 to 512 experts, hidden 1024 to 4096, inter 128 to 2048
+    and 24 to 400 rows an expert, BF16 and FP16 (8 experts of 4096 / 1024, 24
+    rows in BF16: 87.5 against 92.5 us).  Hidden above that, in BF16: fewer than
+    128 w13 workgroups 1.04 to 2.2 (8 experts of 14336 / 512, 24 rows: 207
+    against 95 us); 128 workgroups 1.07 to 1.21 at 24 rows of 5120 to 8192, 0.91
+    to 1.04 at 48, 0.88 to 0.93 at 64, and at 14336 1.25 at 48, 1.05 at 64, 0.95
+    at 110; 256 and more up to 7168 0.85 to 1.03 at 24 rows, less above."""
+    rows = tokens * topk / max(routed_experts, 1)
+    if rows <= 22:
+        return False
+    if hidden <= _ROWS_ANY_HIDDEN:
+        return True
+    workgroups = experts * math.ceil(rows / _TASK_ROWS) * math.ceil(inter / 128)
+    return ((workgroups >= _ROWS_MIN_WORKGROUPS and rows >= hidden / 128)
+            or (workgroups >= _ROWS_FULL_WORKGROUPS and hidden <= _ROWS_FULL_HIDDEN))
+
+
 def rows_task_rows(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
                    w1_scale: torch.Tensor, w2_scale: torch.Tensor, topk: int) -> int:
     """Rows per task of the many-rows path (marlin_moe_rows) for a call, or 0
-    where it does not apply (the staged path's own checks then answer): whole
+    where it cannot run it (the staged path's own checks then answer): whole
     128-column gate / up pairs, at most 1024 experts, 16-byte aligned contiguous
     weights and rows, 32-bit offsets."""
     M, K = hidden_states.shape
@@ -173,7 +207,11 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
         inside = (ids >= 0) & (ids < emap.numel())
         local = torch.where(inside, emap[torch.where(inside, ids, 0).long()], -1).contiguous()
     bs = block_size or choose_block_size(M, topk, E)
-    if path is None and block_size is None and ksplit is None and bs > _DIRECT_MAX_BLOCK:
+    # slots routed to experts held elsewhere take no row here: a map says how
+    # many experts share the call's slots
+    routed_experts = E if expert_map is None else max(E, expert_map.numel())
+    if (path is None and block_size is None and ksplit is None and bs > _DIRECT_MAX_BLOCK
+            and rows_applies(M, topk, K, N, E, routed_experts)):
         task_rows = rows_task_rows(hidden_states, w1, w2, w1_scale, w2_scale, topk)
         if task_rows:
             # the slots grouped by expert in tasks of task_rows rows, each
