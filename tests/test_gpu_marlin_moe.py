@@ -688,3 +688,20 @@ def test_many_rows_run_where_row_lists_are_faster(mm, device, K, N, held, want):
     assert want in ws and not {"table", "part"} - {want} & set(ws)
     expected = M.moe(x, dtype, emap[ids], w, *layer.host)
     assert_close(host_bits(out), expected, dtype, f"K={K} held={held}")
+
+
+def test_many_rows_with_slot_rows_8_byte_aligned(mm, device):
+    """A caller's c3 on an 8-byte boundary: row lists need a 16-byte
+    one, the staged path does not, so the call runs there."""
+    print("c3 off a 16-byte boundary", flush=True)
+    rng = np.random.default_rng(3)
+    E, K, N, T, topk, dtype = 4, 256, 128, 46, 2, M.BF16
+    layer = Layer(rng, E, K, N, dtype, device)
+    ids, w = routing(rng, T, E, topk)
+    x = from_f32(rng.standard_normal((T, K)), dtype)
+    ws = {"c3": torch.empty(T * topk * K + 4, dtype=torch.bfloat16, device=device)[4:]}
+    out = mm[0].fused_marlin_moe(dev_act(x, dtype, device), layer.w1, layer.w2, layer.s1, layer.s2,
+                                 dev(w, device), dev(ids, device), workspace=ws)
+    torch.cuda.synchronize()
+    assert ws["c3"].data_ptr() % 16
+    assert_close(host_bits(out), M.moe(x, dtype, ids, w, *layer.host), dtype, "c3 offset")

@@ -129,11 +129,13 @@ def rows_applies(tokens: int, topk: int, hidden: int, inter: int, experts: int,
 
 
 def rows_task_rows(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
-                   w1_scale: torch.Tensor, w2_scale: torch.Tensor, topk: int) -> int:
+                   w1_scale: torch.Tensor, w2_scale: torch.Tensor, topk: int,
+                   workspace: dict | None = None) -> int:
     """Rows per task of the many-rows path (marlin_moe_rows) for a call, or 0
     where it cannot run it (the staged path's own checks then answer): whole
     128-column gate / up pairs, at most 1024 experts, 16-byte aligned contiguous
-    weights and rows, 32-bit offsets."""
+    weights and rows, 32-bit offsets, 16-byte aligned buffers where the
+    workspace brings them (the staged path takes a c3 8-byte aligned)."""
     M, K = hidden_states.shape
     E, N = w1.size(0), w2.size(1) * 16
     slots = M * topk
@@ -144,6 +146,9 @@ def rows_task_rows(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tens
     tensors = (hidden_states, w1, w2, w1_scale, w2_scale)
     if any(t.data_ptr() % 16 for t in tensors) or any(
             not t.is_contiguous() or t.device != hidden_states.device for t in tensors[1:]):
+        return 0
+    buffers = [(workspace or {}).get(name) for name in ("table", "xp", "h", "c3")]
+    if any(t is not None and t.data_ptr() % 16 for t in buffers):
         return 0
     return _TASK_ROWS
 
@@ -212,7 +217,7 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
     routed_experts = E if expert_map is None else max(E, expert_map.numel())
     if (path is None and block_size is None and ksplit is None and bs > _DIRECT_MAX_BLOCK
             and rows_applies(M, topk, K, N, E, routed_experts)):
-        task_rows = rows_task_rows(hidden_states, w1, w2, w1_scale, w2_scale, topk)
+        task_rows = rows_task_rows(hidden_states, w1, w2, w1_scale, w2_scale, topk, workspace)
         if task_rows:
             # the slots grouped by expert in tasks of task_rows rows, each
             # task's weights dequantized once
