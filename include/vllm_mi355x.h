@@ -94,7 +94,8 @@ int64_t exl3_linear_scratch_rows(int64_t padded_in, int64_t padded_out);
  * The row count above which exl3_linear_out always runs a many-row GEMM.  Up
  * to it: the small-M kernel for 8 rows; above 8, the tile GEMM where it
  * applies (at least 1024 inputs, a 16-byte aligned trellis, a workspace with
- * room), else the small-M kernel in chunks of 8 rows.  The reference's routing
+ * room) and is the faster one (above 16 rows always, from 9 to 16 by the
+ * matrix's size), else the small-M kernel in chunks of 8 rows.  The reference's routing
  * question _exl3_C::linear_prefill_applies (vllm_sm80/kernels/exl3/
  * dense_prefill_tc.py:57-80) answers from it.
  */

@@ -677,3 +677,28 @@ def test_tile_sums_of_few_rows_are_as_exact_as_the_small_kernels(ops, device, pr
         errors.append(float((out.double() - want).pow(2).mean().sqrt()))
     print(f"rms error: tile GEMM {errors[0]:.3g}, chunks {errors[1]:.3g}", flush=True)
     assert errors[0] <= 1.05 * errors[1]
+
+
+# sizes on both sides of the rule for 9 to 16 rows (two small-M passes or the
+# tile GEMM's three launches), its first row above, and fewer than 1024 inputs
+@pytest.mark.parametrize("k,n,rows,tile", [
+    (1024, 1024, 9, False), (1024, 1024, 16, False), (1024, 1024, 17, True), (2048, 3072, 12, False),
+    (2048, 3072, 13, True), (2048, 4608, 9, True), (4096, 256, 10, False), (4096, 256, 11, True),
+    (896, 384, 32, False)])
+def test_few_rows_run_on_the_faster_kernel(ops, device, prefill_switches, k, n, rows, tile):
+    """A call of 9 to 32 rows equals the small-M chunks bit for bit where those
+    are faster; elsewhere the tile GEMM ran: FP32 sums in another order, close
+    to the chunks' and not all the same."""
+    print(f"few rows {k}x{n} rows={rows}", flush=True)
+    rng = np.random.default_rng(k + n + rows)
+    bits_x2, codebook = 8, 2
+    trellis, suh, svh = (_dev(a, device) for a in random_matrix(rng, k, n, bits_x2))
+    x = _dev(random_acts(rng, rows, k, "fp16")[0], device)
+    ws = torch.empty(ops.linear_workspace_size(rows, k, n), dtype=torch.float32, device=device)
+    got, chunks = (torch.empty(rows, n, dtype=torch.float32, device=device) for _ in range(2))
+    ops.linear_out(x, trellis, suh, svh, bits_x2, codebook, k, n, got, ws)
+    prefill_switches[0](1)
+    ops.linear_out(x, trellis, suh, svh, bits_x2, codebook, k, n, chunks, ws)
+    torch.cuda.synchronize()
+    assert torch.equal(got, chunks) != tile
+    _assert_fp32_close(_out_np(got), _out_np(chunks), f"{k}x{n} rows={rows}")

@@ -212,25 +212,38 @@ int64_t partial_elements(const GemvPlan& p, int64_t rows, int64_t cols) { return
 namespace exl3 {
 namespace {
 
-// Calls of 9 to 32 rows of at least this many inputs run on the tile GEMM
-// where the workspace holds its activations and sums: one pass over the
-// weights in three launches instead of up to four passes in as many (20 rows of
-// a 4096 x 14336 matrix at 3 bits: 49.1 us in chunks, 29.1 on the tile GEMM).
-// Shorter matrices keep the chunks, whose workspace is smaller.
+// Whether the tile GEMM is the faster path of a call of 9 to 32 rows: one pass
+// over the weights in three launches instead of up to four passes in as many (20
+// rows of a 4096 x 14336 matrix at 3 bits: 49.1 us in chunks, 28.8 on the tile
+// GEMM).  From 17 rows on (three or four passes) it is at every size measured,
+// 1024 x 1024 to 4096 x 151552 at 2, 3, 4 and 8 bits: 0.32 to 0.81 of the chunks'
+// time.  At 9 to 16 rows two passes stand against three launches: below 9M weights
+// the chunks win, unless K is long (their finish then adds as many partial sums)
+// or the second chunk is more than half full.  us, chunks / tile GEMM, 4 bits:
+// 1024 x 1024 at 9 rows 11.7 / 13.8, at 16 13.7 / 13.9; 2048 x 2048 12.8 / 14.9,
+// 14.8 / 15.0; 2048 x 4096 (8M) at 9 14.2 / 15.2, at 14 15.9 / 15.4; 2048 x 6144
+// at 9 15.8 / 15.4; 4096 x 4096 at 9 18.8 / 16.2; 8192 x 1024 at 9 16.4 / 16.8, at
+// 12 18.4 / 16.9; 5120 x 512 at 9 15.5 / 16.0, at 12 17.7 / 16.1.
+// Matrices of fewer than 1024 inputs keep the chunks, whose workspace is smaller.
 constexpr int64_t kTileMinInputs = 1024;
+bool tile_pays(int64_t rows, int64_t kp, int64_t np) {
+  constexpr int64_t kM = int64_t(1) << 20;
+  if (rows <= kMaxGemvRows || kp < kTileMinInputs) return false;
+  return rows > 2 * kMaxGemvRows || kp * np >= 9 * kM || (rows >= 11 && kp >= 4096) ||
+         (rows >= 13 && kp * np >= 6 * kM);
+}
 // The fixed scratch that dense callers cut their rows to (8M floats): the
 // size function asks for no more than it on the K splits' account, so the
 // rows that fit it do not change.
 constexpr int64_t kFixedScratch = int64_t(8) << 20;
 
-// Whether a call of at most kGemvChunkedRows rows runs on the tile GEMM: more
-// rows than one small-M launch takes, at the activations' full precision, and
-// a workspace that holds every planned split.
+// Whether a call of at most kGemvChunkedRows rows runs on the tile GEMM: where
+// that pays, at the activations' full precision, and with a workspace that holds
+// every planned split.
 bool tile_small(int64_t rows, const void* trellis, int64_t tiles_k, int64_t tiles_n, int64_t bits_x2,
                 int64_t workspace_numel) {
   const int64_t kp = tiles_k * 16, np = tiles_n * 16;
-  return rows > kMaxGemvRows && kp >= kTileMinInputs && !tile_fp16_only() &&
-         tile_applies(trellis, tiles_k, tiles_n, bits_x2, rows) &&
+  return tile_pays(rows, kp, np) && !tile_fp16_only() && tile_applies(trellis, tiles_k, tiles_n, bits_x2, rows) &&
          workspace_numel >= tile_elements(rows, kp, np, plan_tile(rows, kp, np).splits);
 }
 
@@ -263,7 +276,7 @@ extern "C" int64_t exl3_linear_workspace_size(int64_t max_rows, int64_t padded_i
   // (heights of whole 16-row blocks and max_rows itself bound the others)
   for (int64_t r = std::min<int64_t>(max_rows, 16); r > exl3::kMaxGemvRows;
        r = r < max_rows ? std::min(r + 16, max_rows) : 0) {
-    if (r <= exl3::kGemvChunkedRows && padded_in < exl3::kTileMinInputs) continue;
+    if (r <= exl3::kGemvChunkedRows && !exl3::tile_pays(r, padded_in, padded_out)) continue;
     const exl3::TilePlan p = exl3::plan_tile(r, padded_in, padded_out);
     if (p.blocks == exl3::kTileHeight && p.splits == 1) break;  // more rows, more tiles: no splits
     const int64_t least = exl3::tile_elements(r, padded_in);
