@@ -631,3 +631,42 @@ def test_moe_gate_and_up_together_equal_one_after_the_other(ops, device, tile_ro
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     want = O.moe_out(x_host, code, ids, weights, layer.oracle, expert_map, intermediate, out_dtype=code)
     _assert_moe_close(_out_np(outs[0]), _oracle_f32(want, code), f"pair rows={rows}")
+
+
+@pytest.mark.parametrize("hidden", [384, 1152])
+@pytest.mark.parametrize("entry", ["moe_out", "moe_out_v2"])
+def test_moe_pair_with_rates_of_their_own_and_from_the_smallest_hidden_size(ops, device, entry, hidden):
+    """Gate and up in one launch where their rates differ within every expert
+    (moe_out), and from the smallest hidden size that is sized for it: bitwise
+    equal to one after the other (the smallest workspace accepted), and to the
+    oracle at the bar.  Some slots belong to no local expert."""
+    print(f"moe pair entry={entry} hidden={hidden}", flush=True)
+    rng = np.random.default_rng(hidden)
+    intermediate, experts, topk, rows = 256, 5, 2, 37
+    formats = [(6, 2)] if entry == "moe_out_v2" else [(3, 2), (8, 2), (12, 2), (10, 1), (16, 2)]
+    layer = Layer(rng, experts, hidden, intermediate, formats, device)
+    ids = np.stack([rng.permutation(experts + 2)[:topk] for _ in range(rows)])
+    weights = rng.random((rows, topk)).astype(np.float32)
+    expert_map = np.concatenate([np.arange(experts), [-1, -1]]).astype(np.int64)
+    x_host, code, x = _acts(rng, rows, hidden, "bf16", device)
+    a = rows * topk
+    least = (a * (hidden + 3 * intermediate) + 4 + (a + 3) // 4 * 4 + 4 * a
+             + a * max(hidden, intermediate) // 128 + a)
+    sized = ops.moe_workspace_size(rows, hidden, intermediate, topk, experts)
+    assert sized >= least + a * hidden
+    args = (x, _dev(ids, device), _dev(weights, device), layer.ptrs, layer.meta,
+            _dev(expert_map, device), intermediate)
+    outs = []
+    for size in (sized, least):
+        ws = torch.full((size + 64,), float("nan"), dtype=torch.float32, device=device)
+        out = torch.full_like(x, float("nan"))
+        if entry == "moe_out":
+            ops.moe_out(*args, out, ws[:size])
+        else:
+            ops.moe_out_v2(*args, 6, out, ws[:size])
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(ws[size:]).all())
+        outs.append(out)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    want = O.moe_out(x_host, code, ids, weights, layer.oracle, expert_map, intermediate)
+    _assert_moe_close(_out_np(outs[0]), _oracle_f32(want, code), f"pair {entry} hidden={hidden}")

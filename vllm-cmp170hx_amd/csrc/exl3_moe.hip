@@ -106,15 +106,20 @@ struct MoeLayout {
   __host__ __device__ int64_t input_up() const { return (total() + 3) / 4 * 4; }
   __host__ __device__ int64_t total_up() const { return input_up() + assignments * hpad; }
 };
-// Calls sized for gate and up together: at least this hidden size (shorter
-// rows' projections are launch-bound either way), and fewer routed slots than
-// kPairMaxSlots.  Few tasks leave a projection's launch short of workgroups
-// (27 slots of a 7168 / 2048 layer: 240 for gate, 88 us each; both together
-// take about 100): 208 -> 150 us a call there, 542 -> 519 at 576 slots.  Many
-// rows' operands for both projections no longer fit the 256 MB last-level cache
-// between their forming and their use: 20480 slots of 2560 / 640 took 881 us one
-// after the other and 903 together.
-constexpr int64_t kPairMinHidden = 1024;
+// Calls sized for gate and up together: at least this hidden size, and fewer
+// routed slots than kPairMaxSlots.  Few tasks leave a projection's launch short of
+// workgroups (27 slots of a 7168 / 2048 layer: 240 for gate, 88 us each; both
+// together take about 100).  us a call, one after the other / together: 3 tokens of
+// that layer 228 / 161 and 64 tokens 516 / 488, E 64 of 2048 / 768 at 4 bits and 8
+// tokens 83 / 63, E 32 of 896 / 512 56 / 42 at 32 and 84 / 64 at 256 tokens top-4,
+// E 8 of 384 / 256 37 / 28 at 1 and 61 / 45 at 400 tokens top-2.  (Apart, the
+// GEMV's small stages, below, cost layers of hidden sizes under 1024 2 to 7%.)
+// Inputs of two blocks would do; at 256 the workspace keeps its size.  Many rows'
+// operands for both projections no longer fit the 256 MB last-level cache between
+// their forming and their use: at 8000 slots both ways take the same time (896 /
+// 512 206 / 204, 2048 / 768 414 / 417), 20480 slots of 2560 / 640 881 one after the
+// other and 903 together.
+constexpr int64_t kPairMinHidden = 384;
 constexpr int64_t kPairMaxSlots = 8192;
 
 // ---- 1. route ------------------------------------------------------------------
