@@ -753,6 +753,7 @@ __device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeG
   constexpr int kDepth = 4;
   constexpr int kRows = kTaskRows;
   constexpr int kSub = kRows / 8;
+  static_assert(kSub > 2, "the loops of 1, 2 and kSub sub-blocks");
   constexpr int kChunks = 2;  // 16-byte B chunks per thread per stage, at most
   auto& bop = shared.bop;
   auto& rexp = shared.rexp;
@@ -985,14 +986,10 @@ __device__ __forceinline__ void moe_gemv_task(const Routing& routing, const MoeG
   // the loop for the fewest staged sub-blocks (1, 2 or kSub) that hold the
   // task's rows
   auto run = [&](auto aligned_tag) {
-    if constexpr (kSub >= 4) {
-      if (nsub <= 1) {
-        stream(aligned_tag, std::integral_constant<int, 1>{});
-      } else if (nsub <= 2) {
-        stream(aligned_tag, std::integral_constant<int, 2>{});
-      } else {
-        stream(aligned_tag, std::integral_constant<int, kSub>{});
-      }
+    if (nsub <= 1) {
+      stream(aligned_tag, std::integral_constant<int, 1>{});
+    } else if (nsub <= 2) {
+      stream(aligned_tag, std::integral_constant<int, 2>{});
     } else {
       stream(aligned_tag, std::integral_constant<int, kSub>{});
     }

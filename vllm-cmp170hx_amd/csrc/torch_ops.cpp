@@ -35,7 +35,6 @@ decltype(&moe_align_block_size) native_align = nullptr;
 decltype(&marlin_moe_align_permute) native_align_permute = nullptr;
 decltype(&marlin_moe_gemm) native_gemm = nullptr;
 decltype(&marlin_moe_gemm_direct) native_gemm_direct = nullptr;
-decltype(&marlin_moe_act) native_act = nullptr;
 decltype(&marlin_moe_w13_act) native_w13_act = nullptr;
 decltype(&marlin_moe_w2_sum) native_w2_sum = nullptr;
 decltype(&marlin_moe_rows) native_rows = nullptr;
@@ -252,19 +251,10 @@ void marlin_moe(const at::Tensor& x, const at::Tensor& w1, const at::Tensor& w2,
         owners = eids;
         owner_numel = blocks;
       }
-      if (n % 64 == 0) {
-        check_status(native_w13_act(x.const_data_ptr(), dtype, m, x.stride(0), words(w1), s1.const_data_ptr(), experts,
-                                    sorted, sorted_numel, owners, owner_numel, padded, routed, topk, slots, k, 2 * n,
-                                    block_size, ksplit, static_cast<float>(limit), part, act.numel(),
-                                    h.mutable_data_ptr(), n, slots, stream));
-      } else {
-        constexpr int kPartial = 0;
-        check_status(native_gemm(x.const_data_ptr(), dtype, m, x.stride(0), words(w1), s1.const_data_ptr(), experts,
-                                 sorted, sorted_numel, owners, owner_numel, padded, nullptr, topk, slots, k, 2 * n,
-                                 block_size, kPartial, ksplit, part, act.numel(), nullptr, 0, 0, stream));
-        check_status(native_act(part, routed, ksplit, slots, n, static_cast<float>(limit), h.mutable_data_ptr(), dtype,
-                                stream));
-      }
+      check_status(native_w13_act(x.const_data_ptr(), dtype, m, x.stride(0), words(w1), s1.const_data_ptr(), experts,
+                                  sorted, sorted_numel, owners, owner_numel, padded, routed, topk, slots, k, 2 * n,
+                                  block_size, ksplit, static_cast<float>(limit), part, act.numel(),
+                                  h.mutable_data_ptr(), n, slots, stream));
       if (path == 3) {
         check_status(native_w2_sum(h.const_data_ptr(), dtype, slots, n, words(w2), s2.const_data_ptr(), experts, routed,
                                    slots, weights, topk, slots, n, k, block_size, c3.mutable_data_ptr(), k, slots,
@@ -302,7 +292,7 @@ extern "C" int vllm_mi355x_torch_bind(void* library) {
                    find(library, "marlin_moe_align_permute", native_align_permute) &&
                    find(library, "marlin_moe_gemm", native_gemm) &&
                    find(library, "marlin_moe_gemm_direct", native_gemm_direct) &&
-                   find(library, "marlin_moe_act", native_act) && find(library, "marlin_moe_w13_act", native_w13_act) &&
+                   find(library, "marlin_moe_w13_act", native_w13_act) &&
                    find(library, "marlin_moe_w2_sum", native_w2_sum) && find(library, "marlin_moe_rows", native_rows) &&
                    find(library, "moe_sum", native_sum) && find(library, "vllm_mi355x_last_error", native_last_error);
   return all ? 0 : 1;

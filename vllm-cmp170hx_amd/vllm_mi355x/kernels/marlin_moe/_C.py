@@ -117,6 +117,11 @@ def gemm(a, w, s, sorted_ids, expert_ids, ntpp, topk_w, top_k, n_slots, K, N, bl
     _native.check(status)
 
 
+# gemm_direct, permute_act, align_permute, w13_act and w2_sum are single launches of
+# the direct and identity paths, for callers (and tests) that run one step by
+# itself.  A fused call makes its launches and their checks in C++ (fused).
+
+
 def gemm_direct(a_perm, w, s, sorted_ids, expert_ids, ntpp, topk_w, top_k, n_slots, K, N,
                 block_size, mode, ksplit=1, limit=math.inf, part=None, out=None) -> None:
     """marlin_moe_gemm_direct on torch tensors: gemm's contract on k-permuted
