@@ -702,3 +702,41 @@ def test_few_rows_run_on_the_faster_kernel(ops, device, prefill_switches, k, n, 
     torch.cuda.synchronize()
     assert torch.equal(got, chunks) != tile
     _assert_fp32_close(_out_np(got), _out_np(chunks), f"{k}x{n} rows={rows}")
+
+
+# (k, n, rows, K splits planned): 17 and 9 blocks cut into six and three, which
+# fewer splits cut unevenly
+@pytest.mark.parametrize("k,n,rows,planned", [(2176, 256, 64, 6), (2176, 384, 129, 6), (1152, 384, 33, 3)])
+def test_tile_takes_the_splits_a_workspace_holds(ops, device, k, n, rows, planned):
+    """A workspace with room for s copies of the partial sums, 1 < s < planned:
+    s splits run (the sums differ from the other counts' in their last bits),
+    nothing past the workspace is written, every count is within the FP32 bar of
+    the oracle and any two of them within two bars."""
+    print(f"splits of {planned} {k}x{n} rows={rows}", flush=True)
+    rng = np.random.default_rng(k + n + rows)
+    bits_x2, codebook = 6, 2
+    trellis, suh, svh = random_matrix(rng, k, n, bits_x2)
+    x, code = random_acts(rng, rows, k, "fp16")
+    t, u, v, xt = _dev(trellis, device), _dev(suh, device), _dev(svh, device), _dev(x, device)
+    base = (rows * (k + 1) + 3) // 4 * 4
+    assert ops.linear_workspace_size(rows, k, n) >= base + planned * rows * n
+    want = O.linear_out(x, code, trellis, suh, svh, bits_x2, codebook, n, O.FP32)
+    got = []
+    for splits in sorted({1, 2, planned - 1, planned}):
+        # (one float short of another copy)
+        size = base + (splits + 1) * rows * n - 1
+        ws = torch.full((size + 64,), float("nan"), dtype=torch.float32, device=device)
+        out = torch.empty(rows, n, dtype=torch.float32, device=device)
+        ops.linear_out(xt, t, u, v, bits_x2, codebook, k, n, out, ws[:size])
+        torch.cuda.synchronize()
+        used = base + (splits * rows * n if splits > 1 else 0)
+        assert bool(torch.isnan(ws[used:]).all())
+        if splits > 1:
+            assert not bool(torch.isnan(ws[base:used]).any())
+        got.append(_out_np(out))
+        _assert_fp32_close(got[-1], want, f"{splits} splits")
+    rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    for i, a in enumerate(got):
+        for b in got[:i]:
+            assert (a != b).any()
+            assert (np.abs(a.astype(np.float64) - b) <= 2 * (2.0 ** -14 * rms + 2.0 ** -16 * np.abs(want))).all()

@@ -705,3 +705,59 @@ def test_many_rows_with_slot_rows_8_byte_aligned(mm, device):
     torch.cuda.synchronize()
     assert ws["c3"].data_ptr() % 16
     assert_close(host_bits(out), M.moe(x, dtype, ids, w, *layer.host), dtype, "c3 offset")
+
+
+# several experts a thread of the fill kernel, the most it takes, and more than
+# eight 2048-slot parts (its second batch of histograms)
+@pytest.mark.parametrize("E,slots", [(300, 2500), (1024, 3000), (1024, 17000), (5, 17000)])
+def test_rows_path_many_experts_and_parts(mm, device, E, slots):
+    """Row lists over many experts or many slots against the staged path at one
+    K split, bit for bit."""
+    from vllm_mi355x.kernels.marlin_moe import _C
+    print(f"rows E={E} slots={slots}", flush=True)
+    rng = np.random.default_rng(E + slots)
+    K, N, topk, task_rows, dtype = 128, 128, 2, 128, M.BF16
+    layer = Layer(rng, E, K, N, dtype, device)
+    T = slots // topk
+    ids = dev(rng.integers(-1, E, (T, topk)).astype(np.int32), device)
+    w = dev(rng.random((T, topk)).astype(np.float32), device)
+    x = dev_act(from_f32(rng.standard_normal((T, K)), dtype), dtype, device)
+    want = mm[0].fused_marlin_moe(x, layer.w1, layer.w2, layer.s1, layer.s2, w, ids, block_size=64,
+                                  ksplit=1, path="staged")
+    table = torch.full((_C.rows_table(slots, E, task_rows) + 16,), -1, dtype=torch.int32, device=device)
+    act = lambda *shape: torch.full(shape, float("nan"), dtype=x.dtype, device=device)
+    got = act(T, K)
+    _C.fused(x, layer.w1, layer.w2, layer.s1, layer.s2, w, ids, _C.ROWS, task_rows, 1, math.inf,
+             table[:-16], None, None, act(T, K), act(slots, N), act(slots, K), got)
+    torch.cuda.synchronize()
+    assert bool((table[-16:] == -1).all())
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_direct_call_on_a_side_stream_and_its_refusals(mm, device):
+    """The fused operator's direct launches (as its other paths above): another
+    stream, inputs that require gradients, wrong buffers."""
+    print("fused operator direct", flush=True)
+    rng = np.random.default_rng(9)
+    E, K, N, topk, T = 4, 256, 128, 2, 40
+    layer = Layer(rng, E, K, N, M.BF16, device)
+    x = dev_act(from_f32(rng.standard_normal((T, K)), M.BF16), M.BF16, device)
+    ids, w = routing(rng, T, E, topk)
+    args = (layer.w1, layer.w2, layer.s1, layer.s2, dev(w, device), dev(ids, device))
+    kw = dict(path="direct", block_size=32)
+    want = mm[0].fused_marlin_moe(x, *args, **kw)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    ws = {}
+    with torch.cuda.stream(side):
+        got = mm[0].fused_marlin_moe(x.clone().requires_grad_(), *args, workspace=ws, **kw)
+    side.synchronize()
+    assert "xp" in ws and "table" not in ws and "part" not in ws
+    assert not got.requires_grad
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    expected = M.moe(host_bits(x), M.BF16, ids, w, *layer.host)
+    assert_close(host_bits(want), expected, M.BF16, "direct")
+    for bad in ({"h": torch.empty(2 * T * topk, N, dtype=x.dtype, device=device)[::2]},
+                {"xp": torch.empty(T, K, dtype=x.dtype)}, {"ntpp": torch.empty(1, dtype=torch.int32)}):
+        with pytest.raises(RuntimeError):
+            mm[0].fused_marlin_moe(x, *args, workspace=dict(bad), **kw)
