@@ -124,7 +124,12 @@ int exl3_linear_prefill_rows(void);
  * parts (about 22 significant bits, the activation precision of the
  * reference's tensor-core kernels, csrc/exl3/dense_prefill_tc.h:5-12), so
  * the result agrees with the reference's sequential FP32 chain to FP32
- * rounding, not bit for bit.  Above 32 rows a 16-byte aligned trellis runs
+ * rounding, not bit for bit.  The order of those sums, and so a result's last
+ * bits, depend on the matrix, the number of rows of the call (the kernel and
+ * its K splits are chosen by it) and, where it holds fewer than the planned
+ * K splits, on workspace_numel: equal calls with equal sizes give equal bits,
+ * but a row need not give the same bits alone, in a chunk, or with another
+ * workspace size.  Above 32 rows a 16-byte aligned trellis runs
  * on the many-row tile GEMM, any other on the decode-to-LDS prefill GEMM;
  * under exl3_set_tile_precision(1) the tile GEMM rounds each rotated input
  * once to FP16 instead (FP16-operand tolerance, an rms error of about

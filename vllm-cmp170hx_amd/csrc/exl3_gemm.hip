@@ -72,8 +72,8 @@ constexpr int kLdsK = kBK + 8;      // LDS row stride in halves (80 bytes)
 // of a call of few rows: 20 rows of 14336 inputs take 15.4 us with four
 // wavefronts a row (seven groups each) and under 6 with sixteen.
 // Pass 1 finds the row maximum of |t|, pass 2 writes the scaled high parts
-// (and the low parts when `lo`: the GEMM reads them) as dword pairs; groups past the register cache are formed again
-// (the same operations, so the same values).  Inputs past logical_in form
+// (and the low parts when `lo`: the GEMM reads them), 16 bytes a lane; groups past
+// the register cache are formed again (the same operations, so the same values).  Inputs past logical_in form
 // +0, as the reference's zero padding.
 // Half offset of input k within its 32-input step, in the operand order.
 __device__ __forceinline__ int64_t operand_order(int64_t k) {
@@ -457,11 +457,14 @@ std::atomic<int> g_prefill_kernel{0};
 // split in 128-input blocks.  A call whose tiles leave CUs idle splits K until
 // it has about one workgroup per CU, two for tiles of 32 rows (a short step
 // leaves latency for a second workgroup to fill); beyond that the partial sums
-// cost more than they win.  Measured (us per call, 4 bits, 1 / 4 / 8 / 16 / 32
-// splits): 14336 x 4096 at 77 rows (16 tiles) 293 / 84 / 56 / 43 / 54 before
-// the finish read its splits in parallel; 4096 x 4096 at 200 rows (32
-// tiles) 122 / 47 / 38 / 45 / 45; 4096 x 14336 at 20 rows (56 tiles) 76 / 30 /
-// 29 / 31 / 52; at 64 rows 88 / 38 / 38 / 38 / 38.
+// cost more than they win, and a second workgroup on some of the CUs costs more
+// than the shorter ranges win.  us per call at 128 and 256, 256 and 512, 384 and
+// 768, 512 and 1024 workgroups (taller tiles, 32-row tiles): 14336 x 4096, 4 bits,
+// 77 rows 56.7 / 44.9 / 51.0 / 50.7; 8192 x 8192, 4 bits, 100 rows 69.6 / 53.0 /
+// 67.3 / 67.8; 4096 x 4096, 4 bits, 200 rows 45.0 / 39.2 / 45.8 / 45.8; 4096 x
+// 14336, 3 bits, 20 rows 30.5 / 29.7 / 34.5 / 35.3, at 64 rows 51.8 / 37.7 / 42.2 /
+// 38.8; 14336 x 4096, 4 bits, 20 rows 31.0 / 32.2 / 37.5 / 38.7; 1024 x 1024 and
+// 2048 x 2048 within 2% (the two-block minimum sets their splits).
 constexpr int64_t kSplitGrid = 256;
 constexpr int64_t kSplitGridLow = 512;
 constexpr int64_t kSplitMinBlocks = 2;
