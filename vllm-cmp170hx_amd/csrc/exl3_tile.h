@@ -445,16 +445,23 @@ __global__ __launch_bounds__(kTileThreads, tile_occupancy(kBlocks, kBitsX2)) voi
 #pragma unroll
       for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[rb][p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-              ah[rb], b_cur[p][j], kShortChains && kS == 0 ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : acc[rb][p][j], 0, 0, 0);
+        for (int j = 0; j < 2; ++j) {
+          if constexpr (kShortChains && kS == 0) {
+            acc[rb][p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[rb], b_cur[p][j], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+          } else {
+            acc[rb][p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[rb], b_cur[p][j], acc[rb][p][j], 0, 0, 0);
+          }
+        }
       if constexpr (kLo) {
 #pragma unroll
         for (int p = 0; p < 2; ++p)
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
-            f32x4_t& c = kShortChains ? low[kShortChains ? rb : 0][p][j] : acc[rb][p][j];
-            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[rb], b_cur[p][j], c, 0, 0, 0);
+            if constexpr (kShortChains) {
+              low[rb][p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[rb], b_cur[p][j], low[rb][p][j], 0, 0, 0);
+            } else {
+              acc[rb][p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[rb], b_cur[p][j], acc[rb][p][j], 0, 0, 0);
+            }
           }
       }
     });
@@ -474,13 +481,13 @@ __global__ __launch_bounds__(kTileThreads, tile_occupancy(kBlocks, kBitsX2)) voi
   // runs the loop of its height rounded up to 2, 4, 5, 6 or 8 row blocks (3
   // or 4 in a four-block tile).  None branches around an MFMA.
   auto run = [&](auto row_blocks) __attribute__((always_inline)) {
-    auto four_steps = [&](int s) __attribute__((always_inline)) {
-      step(s, std::integral_constant<int, 0>{}, row_blocks);
-      step(s + 1, std::integral_constant<int, 1>{}, row_blocks);
-      step(s + 2, std::integral_constant<int, 2>{}, row_blocks);
-      step(s + 3, std::integral_constant<int, 3>{}, row_blocks);
-    };
     if constexpr (kShortChains) {
+      auto four_steps = [&](int s) __attribute__((always_inline)) {
+        step(s, std::integral_constant<int, 0>{}, row_blocks);
+        step(s + 1, std::integral_constant<int, 1>{}, row_blocks);
+        step(s + 2, std::integral_constant<int, 2>{}, row_blocks);
+        step(s + 3, std::integral_constant<int, 3>{}, row_blocks);
+      };
       auto each = [&](auto&& f) __attribute__((always_inline)) {
 #pragma unroll
         for (int rb = 0; rb < kBlocks; ++rb)
@@ -505,7 +512,12 @@ __global__ __launch_bounds__(kTileThreads, tile_occupancy(kBlocks, kBitsX2)) voi
       }
       each([&](int rb, int p, int j) { acc[rb][p][j] = total[rb][p][j] + low[rb][p][j]; });
     } else {
-      for (int s = 0; s < steps; s += kTileRing) four_steps(s);
+      for (int s = 0; s < steps; s += kTileRing) {
+        step(s, std::integral_constant<int, 0>{}, row_blocks);
+        step(s + 1, std::integral_constant<int, 1>{}, row_blocks);
+        step(s + 2, std::integral_constant<int, 2>{}, row_blocks);
+        step(s + 3, std::integral_constant<int, 3>{}, row_blocks);
+      }
     }
   };
   // A wavefront whose tile columns all lie past the matrix (in the last
