@@ -152,9 +152,9 @@ int exl3_linear_out(const void* x, int x_dtype, int64_t rows, int64_t x_cols,
  * hpad / ipad the hidden / intermediate sizes rounded up to 128,
  * A * (hpad + 3 * ipad) (activations, gate, up and down-input rows) plus the int32
  * routing table (4 + A rounded up to 4 + 4 A) plus A * max(hpad, ipad) / 128
- * int32 scale exponents plus A int32 experts of the sorted rows; from hpad
- * 384 on, also room for calls of fewer than 8192 slots to form gate and up
- * together (the larger of the above and, with A at most 8191, the above
+ * int32 scale exponents plus A int32 experts of the sorted rows; where hpad or
+ * ipad is at least 384, also room for calls of fewer than 8192 slots to form
+ * gate and up together (the larger of the above and, with A at most 8191, the above
  * rounded up to 4 plus A * hpad).  exl3_moe_out accepts less, down to the
  * formula without that room.  0 when local_experts is 0; -1 (with an error
  * message) for negative counts or nonpositive sizes.

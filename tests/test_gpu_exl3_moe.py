@@ -633,16 +633,17 @@ def test_moe_gate_and_up_together_equal_one_after_the_other(ops, device, tile_ro
     _assert_moe_close(_out_np(outs[0]), _oracle_f32(want, code), f"pair rows={rows}")
 
 
-@pytest.mark.parametrize("hidden", [384, 1152])
+@pytest.mark.parametrize("hidden,intermediate", [(384, 256), (1152, 256), (128, 384), (256, 512)])
 @pytest.mark.parametrize("entry", ["moe_out", "moe_out_v2"])
-def test_moe_pair_with_rates_of_their_own_and_from_the_smallest_hidden_size(ops, device, entry, hidden):
+def test_moe_pair_with_rates_of_their_own_and_at_the_smallest_sizes(ops, device, entry, hidden,
+                                                                    intermediate):
     """Gate and up in one launch where their rates differ within every expert
-    (moe_out), and from the smallest hidden size that is sized for it: bitwise
+    (moe_out), and at the smallest sizes that are sized for it: bitwise
     equal to one after the other (the smallest workspace accepted), and to the
     oracle at the bar.  Some slots belong to no local expert."""
-    print(f"moe pair entry={entry} hidden={hidden}", flush=True)
+    print(f"moe pair entry={entry} {hidden}/{intermediate}", flush=True)
     rng = np.random.default_rng(hidden)
-    intermediate, experts, topk, rows = 256, 5, 2, 37
+    experts, topk, rows = 5, 2, 37
     formats = [(6, 2)] if entry == "moe_out_v2" else [(3, 2), (8, 2), (12, 2), (10, 1), (16, 2)]
     layer = Layer(rng, experts, hidden, intermediate, formats, device)
     ids = np.stack([rng.permutation(experts + 2)[:topk] for _ in range(rows)])

@@ -102,24 +102,25 @@ struct MoeLayout {
   // Where the workspace holds it, the up projection's B operands (A x hpad) in
   // a region of their own: gate and up are then formed in one launch and run
   // in one launch, the up rows' exponents in slot 1 of each assignment's
-  // kmax / 128 (so inputs of at least two 128-blocks).
+  // kmax / 128 (so at least two of them).
   __host__ __device__ int64_t input_up() const { return (total() + 3) / 4 * 4; }
   __host__ __device__ int64_t total_up() const { return input_up() + assignments * hpad; }
 };
-// Calls sized for gate and up together: at least this hidden size, and fewer
-// routed slots than kPairMaxSlots.  Few tasks leave a projection's launch short of
+// Calls sized for gate and up together: the larger of the padded hidden and
+// intermediate sizes at least this, and fewer routed slots than kPairMaxSlots.
+// Few tasks leave a projection's launch short of
 // workgroups (27 slots of a 7168 / 2048 layer: 240 for gate, 88 us each; both
 // together take about 100).  us a call, one after the other / together: 3 tokens of
-// that layer 228 / 161 and 64 tokens 516 / 488, E 64 of 2048 / 768 at 4 bits and 8
+// that layer 234 / 167 and 64 tokens 518 / 486, E 64 of 2048 / 768 at 4 bits and 8
 // tokens 83 / 63, E 32 of 896 / 512 56 / 42 at 32 and 84 / 64 at 256 tokens top-4,
-// E 8 of 384 / 256 37 / 28 at 1 and 61 / 45 at 400 tokens top-2.  (Apart, the
-// GEMV's small stages, below, cost layers of hidden sizes under 1024 2 to 7%.)
-// Inputs of two blocks would do; at 256 the workspace keeps its size.  Many rows'
-// operands for both projections no longer fit the 256 MB last-level cache between
-// their forming and their use: at 8000 slots both ways take the same time (896 /
-// 512 206 / 204, 2048 / 768 414 / 417), 20480 slots of 2560 / 640 881 one after the
-// other and 903 together.
-constexpr int64_t kPairMinHidden = 384;
+// E 8 of 384 / 256 37 / 28 at 1 and 61 / 45 at 400 tokens top-2, E 16 of 256 / 1024
+// 63 / 50 at 160.  (Apart, the GEMV's small stages, below, cost narrow layers 2 to
+// 7%.)  Two blocks would do; layers of 256 / 256 keep the smaller workspace, at 1
+// to 2%.  Many rows' operands for both projections no longer fit the 256 MB
+// last-level cache between their forming and their use: at 8000 slots both ways
+// take the same time (896 / 512 206 / 204, 2048 / 768 414 / 417), 20480 slots of
+// 2560 / 640 881 one after the other and 903 together.
+constexpr int64_t kPairMinWidth = 384;
 constexpr int64_t kPairMaxSlots = 8192;
 
 // ---- 1. route ------------------------------------------------------------------
@@ -724,8 +725,8 @@ struct MoeGemvArgs {
 // floats), and the rows' exponents.  A stage is four steps (128 inputs) of up to
 // 16 rows, two steps of up to 32: 16 KB either way, so that registers and not LDS
 // limit a CU's workgroups: five up to 4 bits (with 32 KB, four steps of 32 rows,
-// four).  64 tokens top-8 of 256 + 1 experts of 7168 / 2048 at 3 bits: 507 ->
-// 482 us a call; 200 tokens top-8 of 64 experts of 2048 / 768 at 3 and 4 bits: 156
+// four).  64 tokens top-8 of 256 + 1 experts of 7168 / 2048 at 3 bits: 507-513 ->
+// 482-490 us a call over two runs; 200 tokens top-8 of 64 experts of 2048 / 768 at 3 and 4 bits: 156
 // -> 152.  Six workgroups spill (840 us), and six or seven with tasks of 16 rows
 // decode the larger experts twice (535).
 constexpr int kTaskCols = 2 * kTaskRows;
@@ -1158,7 +1159,7 @@ extern "C" int64_t exl3_moe_workspace_size(int64_t max_rows, int64_t hidden_size
   if (local_experts == 0) return 0;
   const exl3::MoeLayout lay{exl3::padded(hidden_size), exl3::padded(intermediate_size),
                             max_rows * topk};
-  if (lay.hpad < exl3::kPairMinHidden) return lay.total();
+  if (lay.kmax() < exl3::kPairMinWidth) return lay.total();
   // (larger calls' workspaces hold any smaller call's pair too)
   const exl3::MoeLayout pair{lay.hpad, lay.ipad, std::min(lay.assignments, exl3::kPairMaxSlots - 1)};
   return std::max(lay.total(), pair.total_up());
@@ -1334,7 +1335,7 @@ extern "C" int exl3_moe_out(const void* x, int x_dtype, int64_t rows, int64_t hi
     // gate and up: one form and one GEMV launch for both where the
     // workspace holds both projections' inputs, else one after the other
     const int pair =
-        lay.hpad >= exl3::kPairMinHidden && assignments < exl3::kPairMaxSlots && workspace_numel >= lay.total_up() ? 2 : 1;
+        lay.kmax() >= exl3::kPairMinWidth && assignments < exl3::kPairMaxSlots && workspace_numel >= lay.total_up() ? 2 : 1;
     const int64_t in_step = lay.input_up() - lay.input();
     const int64_t out_step = lay.up() - lay.gate();
     for (int p = 0; p < 2; p += pair) {
