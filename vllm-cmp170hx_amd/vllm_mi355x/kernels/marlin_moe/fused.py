@@ -120,7 +120,7 @@ def rows_applies(tokens: int, topk: int, hidden: int, inter: int, experts: int,
     at 110; 256 and more up to 7168 0.85 to 1.03 at 24 rows, less above.
 
     Slots whose ids the caller masked without passing a map count as run here:
-    with seven of eight masked, up to 16 experts of 2048 to 4096 took 0.6 to 1.4
+    with seven of eight masked, up to 16 experts of 2048 to 4096 took 0.6 to 1.6
     of the staged path's time, 32 and more 0.65 to 0.99."""
     rows = tokens * topk / max(routed_experts, 1)
     if rows <= 22:
